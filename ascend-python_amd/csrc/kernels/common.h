@@ -396,8 +396,10 @@ __device__ __forceinline__ void qmm_store(const QmmEpilogue& e, int64_t m, int64
 //                                                   from and runs the whole tile itself (the fallback path)
 //   nzg_sk_dp=<n>                                   NZ prefill stream-K: n whole-tile rounds first
 //   w4nz_wg=<n>                                     NZ decode kernel: workgroups along N
-//   w4nz_nit=<1..8>                                 NZ decode kernel: 128-row superblocks per wave (K/128 must
-//                                                   split evenly into at most 16 waves of them)
+//   w4nz_nit=<1..32>                                NZ decode kernel: 128-row superblocks per wave (up to 8, K/128
+//                                                   splitting evenly into at most 16 waves of them; else the
+//                                                   ragged form)
+//   w4nz_ragged=1                                   NZ decode kernel: the ragged form for every shape
 struct PlanOverride {
     int w4_stream_nwave = 0, w4_stream_nkb = 0, w4_stream_pf = 0;  // 0: the planner's choice
     bool w4_stream_off = false;
@@ -416,6 +418,7 @@ struct PlanOverride {
     int qmm_rev = 1;
     int qmm_small = -1;
     int w4nz_wg = 0, w4nz_nit = 0;
+    bool w4nz_ragged = false;
 };
 const PlanOverride& plan_override();
 // CUs of the current device (cached per device; 0 if it cannot be read)

@@ -333,17 +333,19 @@ __device__ __forceinline__ u32x4 nz8_operand(uint32_t lo, uint32_t hi) {
 // W8: int8 NZ weights (two 1 KB blocks per 128 rows; the operand of 16-bit MFMA
 // step j is rows 16g + 8*(j&1) .. +8 of block j>>1, and its A operand is
 // x[m, 128s + 64*(j>>1) + 16g + 8*(j&1) ..]).
-constexpr int kNzXSlot = 4096;  // bytes of x per superblock and wave: 16 rows x 256 bytes
+// a lane offset past any buffer here (each is below 2^31 bytes): the load returns zeros and reads no memory
+constexpr uint32_t kNzOutside = 0x80000000u;
 
 // s_waitcnt vmcnt(n) for a value known after unrolling; "memory" keeps the LDS reads after it
 __device__ __forceinline__ void wait_vmcnt(int n) {
     switch (n) {
 #define QK_WAIT_CASE(v) \
     case v: asm volatile("s_waitcnt vmcnt(" #v ")" ::: "memory"); break;
-        QK_WAIT_CASE(0) QK_WAIT_CASE(1) QK_WAIT_CASE(2) QK_WAIT_CASE(3) QK_WAIT_CASE(4) QK_WAIT_CASE(5)
-        QK_WAIT_CASE(6) QK_WAIT_CASE(7) QK_WAIT_CASE(8) QK_WAIT_CASE(9) QK_WAIT_CASE(10) QK_WAIT_CASE(11)
-        QK_WAIT_CASE(12) QK_WAIT_CASE(13) QK_WAIT_CASE(14) QK_WAIT_CASE(15) QK_WAIT_CASE(16) QK_WAIT_CASE(17)
-        QK_WAIT_CASE(18) QK_WAIT_CASE(19) QK_WAIT_CASE(20) QK_WAIT_CASE(21) QK_WAIT_CASE(22) QK_WAIT_CASE(23)
+        QK_WAIT_CASE(0) QK_WAIT_CASE(1) QK_WAIT_CASE(2) QK_WAIT_CASE(3) QK_WAIT_CASE(4) QK_WAIT_CASE(5) QK_WAIT_CASE(6) QK_WAIT_CASE(7)
+        QK_WAIT_CASE(8) QK_WAIT_CASE(9) QK_WAIT_CASE(10) QK_WAIT_CASE(11) QK_WAIT_CASE(12) QK_WAIT_CASE(13) QK_WAIT_CASE(14) QK_WAIT_CASE(15)
+        QK_WAIT_CASE(16) QK_WAIT_CASE(17) QK_WAIT_CASE(18) QK_WAIT_CASE(19) QK_WAIT_CASE(20) QK_WAIT_CASE(21) QK_WAIT_CASE(22) QK_WAIT_CASE(23)
+        QK_WAIT_CASE(24) QK_WAIT_CASE(25) QK_WAIT_CASE(26) QK_WAIT_CASE(27) QK_WAIT_CASE(28) QK_WAIT_CASE(29) QK_WAIT_CASE(30) QK_WAIT_CASE(31)
+        QK_WAIT_CASE(32) QK_WAIT_CASE(33) QK_WAIT_CASE(34) QK_WAIT_CASE(35) QK_WAIT_CASE(36) QK_WAIT_CASE(37) QK_WAIT_CASE(38) QK_WAIT_CASE(39)
 #undef QK_WAIT_CASE
     default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
     }
@@ -355,20 +357,32 @@ __device__ __forceinline__ void wait_vmcnt(int n) {
 // contiguous in such a row, so the same loads read it in place: per lane c*K + 16g, per 64-row block
 // 16*K*(n-block) + 64*(K block).  The two 64-row blocks of a superblock are the two halves of each
 // column's 128-byte line, loaded back to back.
-template <int DT, int NB, int NIT, bool HAS_OFF, bool W8, int SDT, bool NK = false>
-__global__ __launch_bounds__(64 * kNzMaxWaves) void w4nz_decode(WqbmmArgs p, int nwg, int nrb) {
+//
+// NIT == 0 is the ragged form: `nit` superblocks per wave, known at run time and not the same for every wave.
+// Wave w takes superblocks w * nit .. + nit.  A superblock past the wave's or past K is issued like any other, so the hand-counted waits stay exact, but with offsets outside the buffers (zeros, no memory
+// access); the fold of one past K is dropped by a select.  An int8 weight whose K is an odd number of 64-row blocks ends
+// in half a superblock: its x and weight lanes past K read zeros the same way.  SUB (ragged form only) is the
+// number of groups in a superblock: 1 (groups of whole superblocks, or one group over all of K) or 2 (64 rows).
+// XQ: x DMAs per superblock, four rows each (4: any row block; 1, ragged form only: M <= 4).  With one, the x slots
+// shrink to a quarter and the ragged form keeps four superblocks in flight in place of two.
+template <int DT, int NB, int NIT, bool HAS_OFF, bool W8, int SDT, bool NK = false, int SUB = 1, int XQ = 4>
+__global__ __launch_bounds__(64 * kNzMaxWaves) void w4nz_decode(WqbmmArgs p, int nwg, int nrb, int nit) {
     typedef Mfma<DT> MM;
+    constexpr bool RAG = NIT == 0;
     constexpr int WL = W8 ? 2 : 1;         // weight loads per block and superblock
-    constexpr int PF = NIT < 2 ? NIT : 2;  // superblocks in flight per wave
+    // superblocks in flight per wave: what its registers hold
+    constexpr int PF = NIT == 1 ? 1 : XQ == 1 && NB * WL <= 4 ? (NB == 4 ? 3 : 4) : 2;
+    constexpr int XSLOT = XQ * 1024;       // bytes of x per superblock and wave: 4 * XQ rows x 256 bytes
     constexpr int SL = PF;                 // x slots and scale rows per wave
-    constexpr int NT = HAS_OFF ? 2 : 1;    // scale rows per superblock (scale, offset)
+    constexpr int NT = HAS_OFF ? 2 : 1;    // scale rows per group (scale, offset)
     constexpr int RL = 2 * NB;             // 16-byte pieces of one row (NB*16 columns)
-    constexpr int GRP = 5 + NB * WL;       // vector-memory loads per superblock: 4 x DMAs, scale rows, weights
-    static_assert(NT * RL <= 64, "one load instruction fetches a superblock's scale rows");
+    constexpr int GRP = XQ + 1 + NB * WL;  // vector-memory loads per superblock: x DMAs, scale rows, weights
+    static_assert(SUB * NT * RL <= 64, "one load instruction fetches a superblock's scale rows");
+    static_assert(SUB == 1 || RAG, "64-row groups run the ragged form");
     // per wave: its x slots, later its partial sums (NB tiles of kNzTilePitch floats)
-    constexpr int WSLOT = SL * kNzXSlot > NB * kNzTilePitch * 4 ? SL * kNzXSlot : NB * kNzTilePitch * 4;
+    constexpr int WSLOT = SL * XSLOT > NB * kNzTilePitch * 4 ? SL * XSLOT : NB * kNzTilePitch * 4;
     __shared__ __attribute__((aligned(16))) char xbuf[kNzMaxWaves * WSLOT];
-    __shared__ __attribute__((aligned(16))) uint16_t srow[kNzMaxWaves][SL][NT][NB * 16];
+    __shared__ __attribute__((aligned(16))) uint16_t srow[kNzMaxWaves][SL][SUB * NT][NB * 16];
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nwave = blockDim.x >> 6;
@@ -378,46 +392,55 @@ __global__ __launch_bounds__(64 * kNzMaxWaves) void w4nz_decode(WqbmmArgs p, int
     const int rb = lid % nrb, wg = lid / nrb;
     const int M = (int)p.M, K = (int)p.K, N = (int)p.N, G = (int)p.group;
     const int NBT = N >> 4, S = K >> 7;
+    const int KB = W8 ? K >> 6 : S;  // 1 KB blocks per block column (int8: 64 rows each)
     // block range of this workgroup (32-bit: (nwg + 1) * NBT < 2^31, checked by the planner)
     const int b0 = (int)((uint32_t)(wg * NBT) / (uint32_t)nwg), b1 = (int)((uint32_t)((wg + 1) * NBT) / (uint32_t)nwg);
-    const int s0 = wave * NIT;
+    const int s0 = wave * (RAG ? nit : NIT);
 
     // x DMA q of a superblock: rows 4q .. 4q+3 of the row block, lane -> (row 4q + lane/16, 16-byte piece
-    // lane%16); rows past M read row M-1 (each output row depends on its own x row only) and are not stored
+    // lane%16).  Rows past M are not stored (each output row depends on its own x row only), so they are
+    // left outside the buffer: zeros and no memory access.
     const __amdgpu_buffer_rsrc_t xr = make_rsrc(p.x, (uint32_t)M * (uint32_t)K * 2u);
-    uint32_t x_dma[4];
+    uint32_t x_dma[XQ];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < XQ; ++q) {
         const int row = rb * 16 + 4 * q + (lane >> 4);
-        x_dma[q] = (uint32_t)(row < M ? row : M - 1) * (uint32_t)K * 2u + 16u * (uint32_t)(lane & 15);
+        x_dma[q] = row < M ? (uint32_t)row * (uint32_t)K * 2u + 16u * (uint32_t)(lane & 15) : kNzOutside;
     }
     char* const xw = xbuf + wave * WSLOT;
     const uint32_t xw_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)xbuf + (uint32_t)(wave * WSLOT);
     static_assert(!NK || W8, "the [N, K] layout is an int8 weight's");
     const __amdgpu_buffer_rsrc_t wr = make_rsrc(p.w, (uint32_t)K * (uint32_t)N / (W8 ? 1u : 2u));
     const uint32_t w_lane = NK ? (uint32_t)c * (uint32_t)K + 16u * (uint32_t)g : (uint32_t)lane * 16u;
-    // lane l < NT*RL fetches 16 bytes of row l / RL (scale, offset) of a superblock's group: columns
-    // 16*b0 + 8*(l % RL) .. +8, clamped into the row (the clamped columns belong to no block of this
-    // workgroup and are never used); the other lanes repeat lane 0's address
-    const int sl_t = lane < NT * RL ? lane / RL : 0;
-    const int sl_col0 = 16 * b0 + 8 * (lane < NT * RL ? lane % RL : 0);
+    // lane l < SUB*NT*RL fetches 16 bytes of row l / RL (scale, offset, of each group of the superblock in
+    // turn): columns 16*b0 + 8*(l % RL) .. +8, clamped into the row (the clamped columns belong to no block of
+    // this workgroup and are never used); the other lanes repeat lane 0's address
+    const int sl_r = lane < SUB * NT * RL ? lane / RL : 0;
+    const int sl_t = sl_r % NT, sl_u = sl_r / NT;
+    const int sl_col0 = 16 * b0 + 8 * (lane < SUB * NT * RL ? lane % RL : 0);
     const int sl_col = sl_col0 < N ? sl_col0 : N - 8;
     const uint16_t* sl_base = static_cast<const uint16_t*>(sl_t == 0 || !HAS_OFF ? p.scale : p.offset) + sl_col;
+    const uint32_t ng = (uint32_t)K / (uint32_t)G;
 
     int blk[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b) blk[b] = b0 + b < b1 ? b0 + b : b1 - 1;
 
     u32x4 wv[SL][NB][WL], sa[SL];
-    // one superblock's loads in a fixed order: 4 x DMAs, the scale rows, the weights (non-temporal)
-    auto issue = [&](int it) {
+    // superblock s0 + it's loads into slot sl, in a fixed order: the x DMAs, the scale rows, the weights
+    // (non-temporal)
+    auto issue = [&](int it, int sl) {
         asm volatile("" ::: "memory");  // the LDS reads of the slot's previous superblock stay before its DMAs
         __builtin_amdgcn_sched_barrier(0);
-        const int s = s0 + it, sl = it % SL;
+        int s = s0 + it;
+        const bool w_in = !RAG || (it < nit && 128 * s < K);
+        const bool x_in = !RAG || (w_in && 128 * s + 8 * (lane & 15) < K);
+        if (RAG) s = w_in ? s : 0;  // the scalar offsets stay inside the buffers
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            dma16(xr, xw_lds + (uint32_t)(sl * kNzXSlot + q * 1024), x_dma[q], (uint32_t)s * 256u);
-        const uint32_t grp = (uint32_t)(s * 128) / (uint32_t)G;
+        for (int q = 0; q < XQ; ++q)
+            dma16(xr, xw_lds + (uint32_t)(sl * XSLOT + q * 1024), x_in ? x_dma[q] : kNzOutside, (uint32_t)s * 256u);
+        uint32_t grp = (uint32_t)(s * 128) / (uint32_t)G + (SUB > 1 ? (uint32_t)sl_u : 0u);
+        if (RAG) grp = grp < ng ? grp : ng - 1;  // past K: read and dropped by the fold
         sa[sl] = *reinterpret_cast<const u32x4*>(sl_base + (size_t)grp * (uint32_t)N);
 #pragma unroll
         for (int b = 0; b < NB; ++b)
@@ -425,14 +448,14 @@ __global__ __launch_bounds__(64 * kNzMaxWaves) void w4nz_decode(WqbmmArgs p, int
             for (int h = 0; h < WL; ++h)
                 wv[sl][b][h] = __builtin_bit_cast(
                     u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                               wr, w_lane,
+                               wr, !RAG || (w_in && WL * s + h < KB) ? w_lane : kNzOutside,
                                NK ? (uint32_t)blk[b] * 16u * (uint32_t)K + (uint32_t)(128 * s + 64 * h)
-                                  : ((uint32_t)blk[b] * (uint32_t)(WL * S) + (uint32_t)(WL * s + h)) * 1024u,
+                                  : ((uint32_t)blk[b] * (uint32_t)KB + (uint32_t)(WL * s + h)) * 1024u,
                                kNonTemporal));
         __builtin_amdgcn_sched_barrier(0);
     };
 #pragma unroll
-    for (int it = 0; it < PF; ++it) issue(it);
+    for (int it = 0; it < PF; ++it) issue(it, it);
 
     const u32x4 ones = {MM::ONES, MM::ONES, MM::ONES, MM::ONES};
     constexpr float BASE = W8 ? 128.0f : MM::BASE;
@@ -440,17 +463,14 @@ __global__ __launch_bounds__(64 * kNzMaxWaves) void w4nz_decode(WqbmmArgs p, int
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[b] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-#pragma unroll
-    for (int it = 0; it < NIT; ++it) {
-        const int sl = it % SL;
-        // superblock it's x DMAs have landed: after them this wave issued its scale rows and weights and
-        // the whole groups of the superblocks up to it + PF - 1
-        const int later = (it + PF - 1 < NIT - 1 ? PF - 1 : NIT - 1 - it);
+    // folds superblock s0 + it, held in slot sl, once its x DMAs have landed: `later` groups of loads were
+    // issued after its own, and after its DMAs this wave issued its scale rows and weights
+    auto consume = [&](int it, int sl, int later) {
         wait_vmcnt(1 + NB * WL + later * GRP);
         // this superblock's scale rows through the wave's LDS slot
-        if (lane < NT * RL) *reinterpret_cast<u32x4*>(&srow[wave][sl][0][0] + 8 * lane) = sa[sl];
+        if (lane < SUB * NT * RL) *reinterpret_cast<u32x4*>(&srow[wave][sl][0][0] + 8 * lane) = sa[sl];
         u32x4 xk[4], wk[NB][WL];
-        const char* xrow = xw + sl * kNzXSlot + c * 256;  // x row c of the row block
+        const char* xrow = xw + sl * XSLOT + (XQ == 4 ? c : c & 3) * 256;  // x row c (XQ == 1: rows past M repeat)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             xk[j] = *reinterpret_cast<const u32x4*>(xrow + (W8 ? 128 * (j >> 1) + 32 * g + 16 * (j & 1) : 64 * j + 16 * g));
@@ -458,28 +478,54 @@ __global__ __launch_bounds__(64 * kNzMaxWaves) void w4nz_decode(WqbmmArgs p, int
         for (int b = 0; b < NB; ++b)
 #pragma unroll
             for (int h = 0; h < WL; ++h) wk[b][h] = wv[sl][b][h];
-        f32x4 xs = {0.f, 0.f, 0.f, 0.f};
+        constexpr int JS = 4 / SUB;  // MFMA steps per group
+        f32x4 xs[SUB];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) xs = MM::mma(xk[j], ones, xs);
+        for (int u = 0; u < SUB; ++u) {
+            xs[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            f32x4 ag = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if constexpr (W8)
-                    ag = MM::mma(xk[j], nz8_operand<DT>(wk[b][j >> 1][2 * (j & 1)], wk[b][j >> 1][2 * (j & 1) + 1]),
-                                 ag);
-                else
-                    ag = MM::mma(xk[j], nz_operand<MM::MAGIC>(wk[b][0][j]), ag);
-            }
-            const float sf = load_half_bits(srow[wave][sl][0][16 * b + c], SDT);
-            const float of = HAS_OFF ? load_half_bits(srow[wave][sl][NT - 1][16 * b + c], SDT) : 0.0f;
-            const float sx = sf * (of - BASE);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[b][r] = __builtin_fmaf(sf, ag[r], __builtin_fmaf(sx, xs[r], acc[b][r]));
+            for (int j = u * JS; j < (u + 1) * JS; ++j) xs[u] = MM::mma(xk[j], ones, xs[u]);
         }
-        // the x reads of slot sl were consumed by the MFMAs above, so its next DMA may land
-        if (it + PF < NIT) issue(it + PF);
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int u = 0; u < SUB; ++u) {
+                f32x4 ag = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int j = u * JS; j < (u + 1) * JS; ++j) {
+                    if constexpr (W8)
+                        ag = MM::mma(xk[j],
+                                     nz8_operand<DT>(wk[b][j >> 1][2 * (j & 1)], wk[b][j >> 1][2 * (j & 1) + 1]), ag);
+                    else
+                        ag = MM::mma(xk[j], nz_operand<MM::MAGIC>(wk[b][0][j]), ag);
+                }
+                const float sf = load_half_bits(srow[wave][sl][u * NT][16 * b + c], SDT);
+                const float of = HAS_OFF ? load_half_bits(srow[wave][sl][u * NT + NT - 1][16 * b + c], SDT) : 0.0f;
+                const float sx = sf * (of - BASE);
+                const bool in = !RAG || 128 * (s0 + it) + (128 / SUB) * u < K;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float v = __builtin_fmaf(sf, ag[r], __builtin_fmaf(sx, xs[u][r], acc[b][r]));
+                    acc[b][r] = in ? v : acc[b][r];
+                }
+            }
+    };
+    // the x reads of a slot are consumed by its MFMAs, so its next DMAs may land right after
+    if constexpr (RAG) {
+        for (int it = 0; it < nit; it += PF)
+#pragma unroll
+            for (int u = 0; u < PF; ++u) {
+                if (it + u >= nit) break;
+                consume(it + u, u, PF - 1);
+                issue(it + u + PF, u);
+            }
+        wait_vmcnt(0);  // the last issues' DMAs, before the slots take the partial sums
+    } else {
+#pragma unroll
+        for (int it = 0; it < NIT; ++it) {
+            consume(it, it % SL, it + PF - 1 < NIT - 1 ? PF - 1 : NIT - 1 - it);
+            if (it + PF < NIT) issue(it + PF, it % SL);
+        }
     }
 
     // partial sums of wave w: NB tiles at xbuf + w * WSLOT; lane (c, g) holds rows 4g..4g+3 of column c of
@@ -873,20 +919,27 @@ __global__ __launch_bounds__(nzg::NT) void w4nz_gemm(WqbmmArgs p, int tiles_m, i
 // 1 beyond; int8 (two loads per block), 3 up to 2 superblocks, 2 for 3, 1 beyond.  Only these
 // (NB, NIT) pairs are built.
 constexpr int nz_max_blocks(int nit, bool w8) {
+    if (nit == 0) return w8 ? 3 : 4;  // the ragged form keeps two superblocks in registers, whatever its length
     return w8 ? (nit <= 2 ? 3 : nit == 3 ? 2 : 1) : (nit <= 3 ? 4 : nit == 4 ? 3 : nit == 5 ? 2 : 1);
 }
 
 struct NzPlan {
     bool ok;
     int nb, nit, nwave, nwg, nrb;
+    bool ragged;
+    int sub;  // groups per superblock
 };
 
 NzPlan nz_plan(const WqbmmArgs& p) {
-    NzPlan z{false, 0, 0, 0, 0, 0};
+    NzPlan z{};
     const int64_t G = p.group == 0 ? p.K : p.group;
     const bool w8 = p.w_dtype == QK_I8_NZ || p.w_dtype == QK_I8_NK;
     if (!(p.w_dtype == QK_I4_NZ || w8) || p.M <= 0 || p.M > 64 || p.N <= 0 || p.K <= 0) return z;
-    if (p.N % 16 != 0 || p.K % 128 != 0 || G <= 0 || G % 128 != 0 || p.K % G != 0) return z;
+    // groups of whole superblocks, halves of one, or one group over all of K
+    if (p.N % 16 != 0 || p.K % (w8 ? 64 : 128) != 0 || G <= 0 || p.K % G != 0) return z;
+    if (G % 128 != 0 && G != 64 && G != p.K) return z;
+    // an [N, K] weight of another K or group is transposed into the workspace (the size query promises that room)
+    if (p.w_dtype == QK_I8_NK && (p.K % 128 != 0 || G % 128 != 0)) return z;
     // 32-bit buffer offsets
     if (p.K * p.N >= ((int64_t)1 << 31) || p.M * p.K * 2 >= ((int64_t)1 << 31) ||
         (p.K / G) * p.N * 2 >= ((int64_t)1 << 31))
@@ -894,24 +947,42 @@ NzPlan nz_plan(const WqbmmArgs& p) {
     if ((uintptr_t)p.x % 16 != 0 || (uintptr_t)p.w % 16 != 0 || (uintptr_t)p.scale % 16 != 0 ||
         (uintptr_t)p.out % 2 != 0 || (p.offset && (uintptr_t)p.offset % 16 != 0))
         return z;
-    const int64_t S = p.K / 128, NBT = p.N / 16;
-    // superblocks per wave: the fewest that give at most 16 waves and split K evenly
-    int nit = 0;
-    const int want = plan_override().w4nz_nit;  // debug override: superblocks per wave
-    for (int t = 1; t <= 8; ++t)
-        if (S % t == 0 && S / t <= kNzMaxWaves && (want == 0 || t == want)) {
-            nit = t;
-            break;
-        }
-    if (nit == 0) return z;
-    z.nit = nit;
-    z.nwave = (int)(S / nit);
+    const int64_t S = (p.K + 127) / 128, NBT = p.N / 16;
+    const PlanOverride& ov = plan_override();  // debug override: superblocks per wave, the ragged form
+    z.sub = G == 64 && p.K != 64 ? 2 : 1;
     z.nrb = (int)((p.M + 15) / 16);
     // blocks per workgroup: what one workgroup per CU needs, within what fits the wave's registers
     // (nz_max_blocks); then as few workgroups as give no workgroup more blocks than that
-    const int cap = nz_max_blocks(nit, w8);
     int64_t nb = (NBT + 255) / 256;
-    if (const int f = plan_override().w4nz_wg) nb = (NBT + f - 1) / f;  // debug override: a workgroup count
+    if (const int f = ov.w4nz_wg) nb = (NBT + f - 1) / f;  // debug override: a workgroup count
+    // superblocks per wave: the fewest that give at most 16 waves and split K evenly, up to 8
+    int nit = 0;
+    if (p.K % 128 == 0 && G != 64 && !ov.w4nz_ragged)
+        for (int t = 1; t <= 8; ++t)
+            if (S % t == 0 && S / t <= kNzMaxWaves && (ov.w4nz_nit == 0 || t == ov.w4nz_nit)) {
+                nit = t;
+                break;
+            }
+    // Even splits of more than two superblocks per wave run the ragged form where it is faster (us, even against
+    // ragged): up to 4 rows, which it gives smaller x slots and more superblocks in flight (K = 14336, N = 4096,
+    // M = 1: 12.1 / 9.7; K = 8192, N = 8192 int8: 17.8 / 15.1), and where the even form's registers hold fewer
+    // blocks than a workgroup per CU needs (M = 16: K = 5120, N = 13696 17.9 / 12.7; K = 8192, N = 28672 36.1 /
+    // 32.7, int8 64.9 / 55.7).  Elsewhere the unrolled even form is ahead (M = 16: K = 8192, N = 3584 9.0 / 10.2,
+    // K = 5120, N = 1536 6.7 / 7.8), also for [N, K] rows (K = 5120, N = 13696, M = 9: 31.5 / 36.7) and for one
+    // row block of an int8 weight on fewer than 16 waves (the same shape, M = 8: 23.6 / 25.0).
+    if (nit > 2 && ov.w4nz_nit == 0) {
+        const bool held = nb <= nz_max_blocks(nit, w8) || p.w_dtype == QK_I8_NK ||
+                          (w8 && z.nrb == 1 && S / nit < kNzMaxWaves);
+        if (p.M <= 4 || !held) nit = 0;
+    }
+    if (nit == 0) {
+        z.ragged = true;
+        nit = (int)((S + kNzMaxWaves - 1) / kNzMaxWaves);
+        if (ov.w4nz_nit > nit) nit = ov.w4nz_nit;
+    }
+    z.nit = nit;
+    z.nwave = (int)((S + nit - 1) / nit);
+    const int cap = nz_max_blocks(z.ragged ? 0 : nit, w8);
     if (nb > cap) nb = cap;
     z.nb = (int)nb;
     z.nwg = (int)((NBT + nb - 1) / nb);
@@ -919,14 +990,14 @@ NzPlan nz_plan(const WqbmmArgs& p) {
     return z;
 }
 
-template <int DT, int NB, int NIT, bool OFF, bool W8, bool NK>
+template <int DT, int NB, int NIT, bool OFF, bool W8, bool NK, int SUB = 1, int XQ = 4>
 hipError_t launch_nz_k(const WqbmmArgs& p, const NzPlan& z, hipStream_t stream) {
     if constexpr (NB <= nz_max_blocks(NIT, W8)) {
         const dim3 grid((uint32_t)(z.nwg * z.nrb)), block((uint32_t)(64 * z.nwave));
         if (p.s_dtype == QK_BF16)
-            w4nz_decode<DT, NB, NIT, OFF, W8, QK_BF16, NK><<<grid, block, 0, stream>>>(p, z.nwg, z.nrb);
+            w4nz_decode<DT, NB, NIT, OFF, W8, QK_BF16, NK, SUB, XQ><<<grid, block, 0, stream>>>(p, z.nwg, z.nrb, z.nit);
         else
-            w4nz_decode<DT, NB, NIT, OFF, W8, QK_F16, NK><<<grid, block, 0, stream>>>(p, z.nwg, z.nrb);
+            w4nz_decode<DT, NB, NIT, OFF, W8, QK_F16, NK, SUB, XQ><<<grid, block, 0, stream>>>(p, z.nwg, z.nrb, z.nit);
         return hipGetLastError();
     }
     return hipErrorInvalidValue;  // not planned (nz_plan caps NB by nz_max_blocks)
@@ -934,6 +1005,13 @@ hipError_t launch_nz_k(const WqbmmArgs& p, const NzPlan& z, hipStream_t stream) 
 
 template <int DT, int NB, bool OFF, bool W8, bool NK>
 hipError_t launch_nz_nit(const WqbmmArgs& p, const NzPlan& z, hipStream_t stream) {
+    if constexpr (!NK)  // an [N, K] weight is planned with whole-superblock groups only
+        if (z.sub == 2)
+            return p.M <= 4 ? launch_nz_k<DT, NB, 0, OFF, W8, NK, 2, 1>(p, z, stream)
+                            : launch_nz_k<DT, NB, 0, OFF, W8, NK, 2>(p, z, stream);
+    if (z.ragged)
+        return p.M <= 4 ? launch_nz_k<DT, NB, 0, OFF, W8, NK, 1, 1>(p, z, stream)
+                        : launch_nz_k<DT, NB, 0, OFF, W8, NK>(p, z, stream);
     switch (z.nit) {
     case 1: return launch_nz_k<DT, NB, 1, OFF, W8, NK>(p, z, stream);
     case 2: return launch_nz_k<DT, NB, 2, OFF, W8, NK>(p, z, stream);
@@ -1149,8 +1227,10 @@ bool nz_chunks_ok(const WqbmmArgs& p) {
 }
 
 size_t w4_nz_workspace(const WqbmmArgs& p, bool stream_k) {
-    if (!plan_override().w4nz_off && nz_plan(p).ok) return 0;
-    if (nz_chunks_ok(p)) return 0;
+    // the decode kernel needs none; with 64-row groups the query keeps reporting the room of the ND form
+    const NzPlan z = plan_override().w4nz_off ? NzPlan{} : nz_plan(p);
+    if (z.ok && z.sub == 1) return 0;
+    if (!z.ok && nz_chunks_ok(p)) return 0;
     if (!plan_override().w4nz_off && nzg_plan(p).ok) return nzg_workspace(p, stream_k);
     const int nd_dtype = p.w_dtype == QK_I4_NZ ? QK_I32 : QK_I8;
     return QK_SPLIT_COUNTER_BYTES + round256(nd_weight_bytes(p)) +
@@ -1158,7 +1238,7 @@ size_t w4_nz_workspace(const WqbmmArgs& p, bool stream_k) {
 }
 
 hipError_t launch_w4_nz_bmm(const WqbmmArgs& p, void* workspace, size_t ws_bytes, hipStream_t stream) {
-    const NzPlan z = plan_override().w4nz_off ? NzPlan{false, 0, 0, 0, 0, 0} : nz_plan(p);
+    const NzPlan z = plan_override().w4nz_off ? NzPlan{} : nz_plan(p);
     if (z.ok)
         return p.x_dtype == QK_BF16 ? launch_nz_dt<QK_BF16>(p, z, stream) : launch_nz_dt<QK_F16>(p, z, stream);
     if (nz_chunks_ok(p)) {

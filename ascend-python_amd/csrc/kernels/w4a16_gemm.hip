@@ -409,10 +409,13 @@ __global__ __launch_bounds__(64 * NWAVE) void w4_stream(WqbmmArgs p, float* __re
     const int k_wave = split * (KW * NKB * 32) + kw * (NKB * 32);
 
     // buffer resources over this wave's rows: lane offsets in VGPRs, row
-    // offsets in SGPRs (no per-load address arithmetic)
+    // offsets in SGPRs (no per-load address arithmetic).  The last split may
+    // reach past K (K is whole 32-row blocks): the lanes of a block past K
+    // load from outside the resources, zeros without a memory access.
     const uint32_t rowbytes = (uint32_t)NW * 4u;
+    const int k_left = K - k_wave < NKB * 32 ? (K - k_wave > 0 ? K - k_wave : 0) : NKB * 32;
     const __amdgpu_buffer_rsrc_t wr =
-        make_rsrc(static_cast<const char*>(p.w) + (size_t)(uint32_t)k_wave * rowbytes, NKB * 32 * rowbytes);
+        make_rsrc(static_cast<const char*>(p.w) + (size_t)(uint32_t)k_wave * rowbytes, (uint32_t)k_left * rowbytes);
     const uint32_t w_lane = (uint32_t)(8 * kg) * rowbytes + (uint32_t)wc * 4u;
     const __amdgpu_buffer_rsrc_t xr = make_rsrc(p.x, (uint32_t)M * (uint32_t)K * 2u);
     const uint32_t x_lane = ((uint32_t)m * (uint32_t)K + (uint32_t)k_wave + 8u * (uint32_t)kg) * 2u;
@@ -429,13 +432,16 @@ __global__ __launch_bounds__(64 * NWAVE) void w4_stream(WqbmmArgs p, float* __re
     SV sv[NPIECE][SVN], ov[NPIECE][SVN];
 #pragma unroll
     for (int pc = 0; pc < NPIECE; ++pc) {
-        const uint32_t g = (uint32_t)(k_wave + pc * PIECE_KB * 32) / (uint32_t)G;
+        const bool in = pc * PIECE_KB * 32 < k_left;  // a piece past K: scale and offset 0, so its fold adds 0
+        const uint32_t g = in ? (uint32_t)(k_wave + pc * PIECE_KB * 32) / (uint32_t)G : 0u;
         const size_t goff = (size_t)g * (uint32_t)N * 2u;
 #pragma unroll
         for (int v = 0; v < SVN; ++v) {
             const size_t o = goff + s_lane + (size_t)v * sizeof(SV);
             sv[pc][v] = *reinterpret_cast<const SV*>(static_cast<const char*>(p.scale) + o);
             if (HAS_OFF) ov[pc][v] = *reinterpret_cast<const SV*>(static_cast<const char*>(p.offset) + o);
+            if (!in) sv[pc][v] = (SV)0u;
+            if (HAS_OFF && !in) ov[pc][v] = (SV)0u;
         }
     }
     constexpr int SL = PF + 1;
@@ -445,20 +451,24 @@ __global__ __launch_bounds__(64 * NWAVE) void w4_stream(WqbmmArgs p, float* __re
         // the scheduler must not interleave blocks: a later block's load moved
         // ahead, or its use moved up, turns the in-order wait into a drain
         __builtin_amdgcn_sched_barrier(0);
-        xa[kb % SL] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, x_lane, kb * 64, 0));
+        constexpr uint32_t kOutside = 0x80000000u;  // past any buffer here (each is below 2^31 bytes)
+        const bool in = kb * 32 < k_left;
+        const uint32_t wl = in ? w_lane : kOutside;
+        xa[kb % SL] = __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, in ? x_lane : kOutside, in ? kb * 64 : 0, 0));
 #pragma unroll
         for (int r = 0; r < 8; ++r) {
-            const uint32_t ro = (uint32_t)(kb * 32 + r) * rowbytes;
+            const uint32_t ro = in ? (uint32_t)(kb * 32 + r) * rowbytes : 0u;
             if constexpr (LW == 4) {
-                const u32x4 d = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, w_lane, ro, 0));
+                const u32x4 d = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, wl, ro, 0));
 #pragma unroll
                 for (int e = 0; e < 4; ++e) wv[kb % SL][e][r] = d[e];
             } else if constexpr (LW == 2) {
-                const u32x2 d = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(wr, w_lane, ro, 0));
+                const u32x2 d = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(wr, wl, ro, 0));
                 wv[kb % SL][0][r] = d[0];
                 wv[kb % SL][1][r] = d[1];
             } else {
-                wv[kb % SL][0][r] = __builtin_amdgcn_raw_buffer_load_b32(wr, w_lane, ro, 0);
+                wv[kb % SL][0][r] = __builtin_amdgcn_raw_buffer_load_b32(wr, wl, ro, 0);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -1462,14 +1472,14 @@ StreamPlan stream_plan(const WqbmmArgs& p) {
     const int64_t G = p.group == 0 ? p.K : p.group;
     const bool w8 = p.w_dtype == QK_I8;
     if (!(p.w_dtype == QK_I32 || (w8 && p.N % 4 == 0)) || p.M <= 0 || p.M > 16 || p.N <= 0 || p.K <= 0) return s;
-    if (G <= 0 || p.K % G != 0 || !(G % 128 == 0 || G == 32 || G == 64)) return s;
+    if (G <= 0 || p.K % G != 0 || p.K % 32 != 0 || !(G % 128 == 0 || G == 32 || G == 64 || G == p.K)) return s;
     if (p.K * (w8 ? p.N : p.N / 2) >= ((int64_t)1 << 31) || p.M * p.K * 2 >= ((int64_t)1 << 31) ||
         (p.K / G) * p.N * 2 >= ((int64_t)1 << 31))
         return s;
     if (((uintptr_t)p.x | (uintptr_t)p.scale) % 16 != 0 || (uintptr_t)p.out % 8 != 0 || (uintptr_t)p.w % 4 != 0 ||
         (p.offset && (uintptr_t)p.offset % 16 != 0))
         return s;
-    s.piece_kb = G >= 128 ? 4 : (int)(G / 32);
+    s.piece_kb = G == 32 || G == 64 ? (int)(G / 32) : 4;  // one group over a short K is one piece too
     s.wpl = 16;
     s.nwave = 16;
     s.nkb = 4;
@@ -1498,8 +1508,9 @@ StreamPlan stream_plan(const WqbmmArgs& p) {
         int wpl = ov.w4_stream_wpl;
         if (wpl == 0 && s.piece_kb == 4) {
             const int64_t strips = (p.N + 255) / 256;
-            if (p.N % 16 == 0 && p.K % 1024 == 0 && strips * (p.K / 1024) <= 512) wpl = 64;
-            else if (p.N % 8 == 0 && p.K % 512 == 0) wpl = 32;
+            const bool even = p.K % 512 == 0;  // else the last split reaches past K
+            if (p.N % 16 == 0 && (p.K % 1024 == 0 || !even) && strips * ((p.K + 1023) / 1024) <= 512) wpl = 64;
+            else if (p.N % 8 == 0) wpl = 32;
         }
         if (s.piece_kb == 4 && (wpl == 32 || wpl == 64) && p.N % (wpl / 4) == 0) {
             s.wpl = wpl;
@@ -1517,14 +1528,13 @@ StreamPlan stream_plan(const WqbmmArgs& p) {
         s.pf = ov.w4_stream_pf == 3 ? 3 : 2;
     }
     const int halves = (w8 ? 64 : 32) / s.wpl;
-    int kw = s.nwave / halves;
-    const int rows = s.nkb * 32;
+    const int rows = s.nkb * 32, kw_full = s.nwave / halves;
+    int kw = kw_full;
     while (kw > 1 && p.K % (kw * rows) != 0) kw >>= 1;  // fewer K ranges when K is short
-    if (p.K % (kw * rows) != 0) return s;
+    // no instantiated shape splits K evenly: the last split reaches past K (its waves there read nothing)
+    if (p.K % (kw * rows) != 0 || (kw * halves != 8 && kw * halves != 16) || (w8 && kw != kw_full)) kw = kw_full;
     s.nwave = kw * halves;
-    if (s.nwave != 8 && s.nwave != 16) return s;  // the instantiated shapes
-    if (w8 && s.nwave != (s.wpl == 16 ? 16 : 8)) return s;
-    s.nsplit = (int)(p.K / (kw * rows));
+    s.nsplit = (int)((p.K + kw * rows - 1) / (kw * rows));
     s.nstrip = (int)((p.N + 255) / 256);
     if (s.nsplit > 1 && (int64_t)s.nsplit * p.M * p.N * 4 > ((int64_t)256 << 20)) return s;
     s.ok = (int64_t)s.nstrip * s.nsplit < ((int64_t)1 << 31);

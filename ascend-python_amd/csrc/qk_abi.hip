@@ -98,8 +98,10 @@ bool parse_plan(const char* spec, PlanOverride& o) {
             r.qmm_small = std::atoi(v.c_str());
         } else if (k == "w4nz_wg" && std::sscanf(v.c_str(), "%d", &a) == 1 && a >= 1 && a <= 65536) {
             r.w4nz_wg = a;
-        } else if (k == "w4nz_nit" && std::sscanf(v.c_str(), "%d", &a) == 1 && a >= 1 && a <= 8) {
+        } else if (k == "w4nz_nit" && std::sscanf(v.c_str(), "%d", &a) == 1 && a >= 1 && a <= 32) {
             r.w4nz_nit = a;
+        } else if (k == "w4nz_ragged" && v == "1") {
+            r.w4nz_ragged = true;
         } else if (k == "skinny_pf" && (v == "1" || v == "2" || v == "3")) {
             r.skinny_pf = std::atoi(v.c_str());
         } else if (k == "skinny_splits" && std::sscanf(v.c_str(), "%d", &a) == 1 && a >= 1 && a <= 64 &&
