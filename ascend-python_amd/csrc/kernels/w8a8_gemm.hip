@@ -19,6 +19,10 @@
 namespace qk {
 namespace {
 
+// a lane offset past every operand range here (each ends below it): the load returns zeros and reads no memory.
+// The range check covers the lane offset alone, not the scalar one.
+constexpr uint32_t kOutside = 0xffffff00u;
+
 constexpr int kThreads = 256;
 constexpr int BK = 64;        // K bytes per step == K of one i8 MFMA
 constexpr int LDS_ROW = 80;   // padded row stride (bytes) of the LDS tiles
@@ -295,7 +299,7 @@ __device__ __forceinline__ void load_epi_ops(const QmmArgs& p, EpiOps<TM>& o, in
 // hold BM x (2*BN + 16) bytes) so the global stores are 16-byte and
 // row-contiguous.  acc[i][j] holds rows wm*WMR + 16i + 4(lane>>4) + r, column
 // wn*128 + 16j + (lane&15) of the tile (the MFMA 16x16 output layout).
-template <int OUT, int TM, int NT, bool FULL>
+template <int OUT, int TM, int NT, bool FULL, bool RAG = false>
 __device__ __forceinline__ void big_epilogue(const QmmArgs& p, const i32x4 (&acc)[TM][8], const EpiOps<TM>& ops,
                                              int8_t* smem, int64_t m0, int64_t n0, int wm, int wn, int lane, int tid,
                                              int split, int nsplit, int32_t* __restrict__ partial) {
@@ -304,6 +308,7 @@ __device__ __forceinline__ void big_epilogue(const QmmArgs& p, const i32x4 (&acc
     const int fr = lane & 15, g = lane >> 4;
     if (FULL && nsplit > 1) {  // exact int32 partial sums of this K range
         int32_t* dst = partial + (int64_t)split * p.M * p.N;
+        const int cols = RAG ? (int)(p.N - n0 - wn * 128 - fr) : 128;  // columns inside N from this lane's first on
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -312,7 +317,8 @@ __device__ __forceinline__ void big_epilogue(const QmmArgs& p, const i32x4 (&acc
                 if (m >= p.M) continue;  // the last row tile of a ragged M
                 const int64_t ro = m * p.N + n0 + wn * 128 + fr;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) dst[ro + 16 * j] = acc[i][j][r];
+                for (int j = 0; j < 8; ++j)
+                    if (16 * j < cols) dst[ro + 16 * j] = acc[i][j][r];
             }
         return;
     }
@@ -360,6 +366,7 @@ __device__ __forceinline__ void big_epilogue(const QmmArgs& p, const i32x4 (&acc
             const int q = tid + it * NT;
             const int row = q / CPRO, c = q % CPRO;
             if (m0 + row >= p.M) break;  // rows past a ragged M (q grows with the row)
+            if (RAG && n0 + 8 * c >= p.N) continue;  // the last column tile of a ragged N (a multiple of 8)
             const i32x4 v = *reinterpret_cast<const i32x4*>(smem + row * ROWB + 16 * c);
             // written once and not read again here: non-temporal, past the operand lines in the L2
             __builtin_nontemporal_store(v, reinterpret_cast<i32x4*>(static_cast<uint16_t*>(e.out) + (m0 + row) * e.ldo +
@@ -646,8 +653,13 @@ constexpr int A_BASE = NST * B_ST;      // A slots follow the weight stages
 constexpr int OUT_BYTES = BM * (2 * BN + 16);
 constexpr int RING = NST * B_ST + NSA * A_SL;  // 160 KB: all of the CU's LDS
 constexpr int SMEM = RING > OUT_BYTES ? RING : OUT_BYTES;
-
 }  // namespace dm
+
+// qmm_dma's K range per split: whole four-stage rings (256 K), the last split possibly reaching past K
+__host__ __device__ __forceinline__ int64_t dma_k_len(int64_t K, int nsplit) {
+    constexpr int64_t ring = dm::BK * dm::NST;
+    return ((K + ring - 1) / ring + nsplit - 1) / nsplit * ring;
+}
 
 // BMX = 128 (K splits only): 128-row tiles, so a shape with few 256-row tiles needs half the K splits (and half
 // the int32 partials) to fill the CUs.  Waves then own 32 x 128 (two row tiles), an A slot is 16 KB, and each
@@ -660,7 +672,12 @@ constexpr int SMEM = RING > OUT_BYTES ? RING : OUT_BYTES;
 // rev_from (> 0; the CU count, or INT_MAX for none): workgroups in odd rounds of rev_from walk their K range
 // backwards.  A second-round workgroup takes the next column tiles of the same row blocks on its XCD, so it
 // starts on the K stages the first round read last, which are still in that XCD's L2.
-template <int BL, int OUT, int BMX = 256>
+// RAG: N is not whole column tiles or K not whole rings per split (the last column tile, or the last split's K range,
+// is partly outside).  A reads zeros past K, so whatever the weight reads there adds nothing, and the weight's
+// whole offset is in the loads' voff, so the range check keeps every load inside the operand: blocks, rows and K
+// past the edge read as zeros or, where they fall into the next row or block, as values that meet a zero of A or
+// are not stored.  An instance of its own, since these selects cost the even shapes 1-4 %.
+template <int BL, int OUT, int BMX = 256, bool RAG = false>
 __global__ __launch_bounds__(dm::NT) void qmm_dma(QmmArgs p, int tiles_m, int tiles_n, int nsplit,
                                                   int32_t* __restrict__ partial, int rev_from) {
     using namespace dm;
@@ -689,7 +706,7 @@ __global__ __launch_bounds__(dm::NT) void qmm_dma(QmmArgs p, int tiles_m, int ti
     const int tn = (bid % per_group) / gm;
     const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * (SWI ? BN / 2 : BN);
     const int64_t n_up = SWI ? p.N / 2 + n0 : 0;  // SWI: the tile's first up column
-    const int64_t k_len = p.K / nsplit;
+    const int64_t k_len = RAG ? dma_k_len(p.K, nsplit) : p.K / nsplit;
     const uint32_t k_base = (uint32_t)(split * k_len);
 
     const int tid = threadIdx.x;
@@ -708,16 +725,17 @@ __global__ __launch_bounds__(dm::NT) void qmm_dma(QmmArgs p, int tiles_m, int ti
     // an NZ column block: BN/16 consecutive n-blocks of K/64 1 KB blocks, BN * K contiguous bytes
     // SWI: the whole NZ weight (blocks addressed per wave), or the [K,N] rows from the gate columns on, whose
     // chunks 8..15 are moved to the up columns (I - 128 bytes further)
+    const int64_t cols = !RAG || p.N - n0 >= BN ? BN : p.N - n0;  // columns of this tile inside N
     const __amdgpu_buffer_rsrc_t rsB = B_NZ   ? (SWI ? make_rsrc(p.b, (uint32_t)(p.N * p.K))
-                                                     : make_rsrc(p.b + n0 * p.K, (uint32_t)(BN * p.K)))
-                                       : B_KN ? make_rsrc(p.b + n0, (uint32_t)((p.K - 1) * p.sbk + (SWI ? p.N / 2 + BN / 2 : BN)))
-                                              : make_rsrc(p.b + n0 * p.sbn, (uint32_t)(BN * p.sbn));
+                                                     : make_rsrc(p.b + n0 * p.K, (uint32_t)(cols * p.K)))
+                                       : B_KN ? make_rsrc(p.b + n0, (uint32_t)((p.K - 1) * p.sbk + (SWI ? p.N / 2 + BN / 2 : cols)))
+                                              : make_rsrc(p.b + n0 * p.sbn, (uint32_t)(RAG ? (cols - 1) * p.sbn + p.K : BN * p.sbn));
     const uint32_t kblocks = (uint32_t)(p.K >> 6);
     const uint32_t lda = (uint32_t)p.lda, ldb = (uint32_t)(B_KN ? p.sbk : p.sbn);
     // A [row][128 B]: one instruction = 8 rows 8b..8b+7; lane l -> row l>>3, LDS chunk l&7, and
     // (r>>1)&7 = 4*(b&1) + (l>>4)
-    const uint32_t va0 = (uint32_t)(lane >> 3) * lda + 16u * (uint32_t)((lane & 7) ^ (lane >> 4));
-    const uint32_t va1 = (uint32_t)(lane >> 3) * lda + 16u * (uint32_t)((lane & 7) ^ (4 + (lane >> 4)));
+    const uint32_t ca0 = 16u * (uint32_t)((lane & 7) ^ (lane >> 4)), ca1 = ca0 ^ 64u;  // K byte of the lane's chunk
+    const uint32_t va0 = (uint32_t)(lane >> 3) * lda + ca0, va1 = (uint32_t)(lane >> 3) * lda + ca1;
     // [N,K] weight [row][64 B]: one instruction = 16 rows; lane l -> row l>>2, LDS chunk l&3
     const uint32_t vrk_b = (uint32_t)(lane >> 2) * ldb + 16u * (uint32_t)((lane & 3) ^ ((lane >> 3) & 3));
     // [k][256 B]: one instruction = 4 rows 4b..4b+3 (b = 4*gw + i); lane l -> row l>>4, LDS chunk l&15, and
@@ -747,9 +765,11 @@ __global__ __launch_bounds__(dm::NT) void qmm_dma(QmmArgs p, int tiles_m, int ti
                 dma16(rsB, sbase + st * B_ST + b * 1024, (nb * kblocks + (k0 >> 6)) * 1024u + 16u * lane, 0u);
             }
             else if constexpr (B_KN)
-                dma16(rsB, sbase + st * B_ST + b * 1024, (i & 1) ? vkn1 : vkn0, (k0 + 4u * b) * ldb);
+                dma16(rsB, sbase + st * B_ST + b * 1024, ((i & 1) ? vkn1 : vkn0) + (RAG ? (k0 + 4u * b) * ldb : 0u),
+                      RAG ? 0u : (k0 + 4u * b) * ldb);
             else
-                dma16(rsB, sbase + st * B_ST + b * 1024, vrk_b, (uint32_t)(16 * b) * ldb + k0);
+                dma16(rsB, sbase + st * B_ST + b * 1024, vrk_b + (RAG ? (uint32_t)(16 * b) * ldb + k0 : 0u),
+                      RAG ? 0u : (uint32_t)(16 * b) * ldb + k0);
         }
     };
     // group 0 issues A: rows 128h..128h+127 of range r (K bytes 128r..128r+127 of this split) into slot
@@ -759,10 +779,12 @@ __global__ __launch_bounds__(dm::NT) void qmm_dma(QmmArgs p, int tiles_m, int ti
         const int rs = rev ? nr - 1 - rs0 : rs0;
         const uint32_t lds = sbase + A_BASE + (uint32_t)(r % NSA) * A_SL;
         const uint32_t k0 = k_base + (uint32_t)rs * A_KB;
+        const bool in0 = !RAG || k0 + ca0 < (uint32_t)p.K, in1 = !RAG || k0 + ca1 < (uint32_t)p.K;
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
             const int b = 4 * NA * h + NA * gw + i;  // rows 8b .. 8b+7 (b & 1 == i & 1)
-            dma16(rsA, lds + b * 1024, ((i & 1) ? va1 : va0) + (uint32_t)(8 * b) * lda, k0);
+            const uint32_t v = ((i & 1) ? va1 : va0) + (uint32_t)(8 * b) * lda;
+            dma16(rsA, lds + b * 1024, ((i & 1) ? in1 : in0) ? v : kOutside, k0);
         }
     };
 
@@ -854,11 +876,11 @@ __global__ __launch_bounds__(dm::NT) void qmm_dma(QmmArgs p, int tiles_m, int ti
         if (nsplit != 1) return;
         const QmmEpilogue& e = p.epi;
         const int64_t n = n0 + 4 * lane, m = m0 + 4 * lane;  // 64 lanes x 16 B: 256 columns or rows
-        if (wave == 0 && e.scale && e.scale_per_ch) warm = e.scale[n];
+        if (wave == 0 && e.scale && e.scale_per_ch && (!RAG || n < p.N)) warm = e.scale[n];
         else if (wave == 1 && e.pertoken && m < p.M) warm = e.pertoken[m];
         else if (wave == 2 && e.bias_dtype) {
             const int es = (e.bias_dtype == QK_F32 || e.bias_dtype == QK_I32) ? 4 : 2;
-            if (16 * lane < 256 * es) warm = *(const float*)((const char*)e.bias + n0 * es + 16 * lane);
+            if (16 * lane < cols * es) warm = *(const float*)((const char*)e.bias + n0 * es + 16 * lane);
         }
     };
     if (pg == 0) {
@@ -908,7 +930,7 @@ __global__ __launch_bounds__(dm::NT) void qmm_dma(QmmArgs p, int tiles_m, int ti
     } else {
         EpiOps<TM> ops;
         if (nsplit == 1) load_epi_ops<TM>(p, ops, m0, n0, wm, wn, lane);
-        big_epilogue<OUT, TM, NT, true>(p, acc, ops, smem, m0, n0, wm, wn, lane, tid, split, nsplit, partial);
+        big_epilogue<OUT, TM, NT, true, RAG>(p, acc, ops, smem, m0, n0, wm, wn, lane, tid, split, nsplit, partial);
     }
 }
 
@@ -922,6 +944,9 @@ __global__ __launch_bounds__(dm::NT) void qmm_dma(QmmArgs p, int tiles_m, int ti
 // epilogue as every other path.
 namespace sk {
 constexpr int BN = 256, BK = 128;
+__host__ __device__ __forceinline__ int64_t sk_k_len(int64_t K, int64_t nsplit) {
+    return (K / BK + nsplit - 1) / nsplit * BK;
+}
 }
 
 template <bool B_KN, int MT, bool FINAL, int PF = 1>
@@ -940,7 +965,8 @@ __global__ __launch_bounds__(kThreads) void qmm_skinny(QmmArgs p, int tiles_n, i
     const int split = (blk / tiles_n) % nsplit;
     const int tm = blk / (tiles_n * nsplit);
     const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * sk::BN;
-    const int64_t ks = p.K / nsplit, kbeg = (int64_t)split * ks;
+    // whole stages per split, the last split shorter where they do not divide evenly
+    const int64_t ks = sk::sk_k_len(p.K, nsplit), kbeg = (int64_t)split * ks;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1001,7 +1027,7 @@ __global__ __launch_bounds__(kThreads) void qmm_skinny(QmmArgs p, int tiles_n, i
         for (int j = 0; j < 4; ++j) acc[i][j] = (i32x4){0, 0, 0, 0};
     const int tr_base = kn_off(16 * g + (fr >> 1), 0) + 8 * (fr & 1);
 
-    const int64_t nk = ks / sk::BK;
+    const int64_t nk = (p.K - kbeg < ks ? p.K - kbeg : ks) / sk::BK;
     gload(kbeg, 0);
     lstore(0, 0);
 #pragma unroll
@@ -1159,7 +1185,9 @@ __device__ __forceinline__ void store8(const QmmEpilogue& e, int64_t m, int64_t 
 // SPLIT: the grid holds nsplit workgroups per tile, each over K / nsplit; each stores its exact int32 tile
 // sums device-coherently to partial[tile][split], and the last to arrive (splitk_last) adds the splits in
 // split order and applies the epilogue.
-template <int BL, int BM, int BN, int NW, int PD, int OUT, bool SPLIT>
+// RAG: K is not whole stages or N not whole column blocks; an instance of its own, since its selects cost the even
+// [K,N] shapes up to a fifth (M = 64, N = K = 8192: 28.6 -> 34.2 us).
+template <int BL, int BM, int BN, int NW, int PD, int OUT, bool SPLIT, bool RAG = false>
 __global__ __launch_bounds__(64 * NW + (PD > 0 ? 64 : 0)) void qmm_mid(QmmArgs p, int tiles_m, int nsplit,
                                                                      int32_t* __restrict__ partial,
                                                                      uint64_t* __restrict__ ctr, uint64_t tag) {
@@ -1189,29 +1217,35 @@ __global__ __launch_bounds__(64 * NW + (PD > 0 ? 64 : 0)) void qmm_mid(QmmArgs p
     const uint32_t lda = (uint32_t)p.lda, ldb = (uint32_t)(B_KN ? p.sbk : p.sbn);
     const __amdgpu_buffer_rsrc_t rsA = make_rsrc(p.a + m0 * p.lda, (uint32_t)((rows - 1) * p.lda + p.K));
     // an NZ column block is BN/16 consecutive n-blocks of K/64 blocks each: BN * K contiguous bytes
-    const __amdgpu_buffer_rsrc_t rsB = B_NZ   ? make_rsrc(p.b + n0 * p.K, (uint32_t)(BN * p.K))
+    const int64_t cols = RAG && p.N - n0 < BN ? p.N - n0 : BN;  // fewer in the last block of a ragged N (not [K,N])
+    const __amdgpu_buffer_rsrc_t rsB = B_NZ   ? make_rsrc(p.b + n0 * p.K, (uint32_t)(cols * p.K))
                                        : B_KN ? make_rsrc(p.b + n0, (uint32_t)((p.K - 1) * p.sbk + BN))
-                                              : make_rsrc(p.b + n0 * p.sbn, (uint32_t)((BN - 1) * p.sbn + p.K));
+                                              : make_rsrc(p.b + n0 * p.sbn, (uint32_t)((cols - 1) * p.sbn + p.K));
     const uint32_t kblocks = (uint32_t)(p.K >> 6);  // NZ: 1 KB blocks per n-block
+    const uint32_t K = (uint32_t)p.K;
     // NZ DMA: instruction b copies block (n-block b/4 of the column block, K block 4*stage + b%4); the whole
     // offset goes in voff
     auto voff_nz = [&](int b, uint32_t k0) {
         return ((uint32_t)(b >> 2) * kblocks + (k0 >> 6) + (uint32_t)(b & 3)) * 1024u + 16u * (uint32_t)lane;
     };
+    // The last stage of a ragged K: what lies past K is loaded from outside (zeros; an NZ block past K may be
+    // the next n-block's, which meets a zero of A).
     // [row][256 B] DMA (A, [N,K] weight): an instruction covers rows 4b..4b+3; lane l -> row 4b + (l>>4),
-    // LDS chunk l&15, global chunk (l&15) ^ (row&15)
-    auto voff_rk = [&](int b, uint32_t ld) {
+    // LDS chunk l&15, global chunk (l&15) ^ (row&15); k0, the stage's first K byte, goes in the scalar offset
+    auto voff_rk = [&](int b, uint32_t ld, uint32_t k0) {
         const int row = 4 * b + (lane >> 4);
-        return (uint32_t)row * ld + 16u * (uint32_t)((lane & 15) ^ (row & 15));
+        const uint32_t ch = 16u * (uint32_t)((lane & 15) ^ (row & 15));
+        return !RAG || k0 + ch < K ? (uint32_t)row * ld + ch : kOutside;
     };
     // [k][BN B] DMA ([K,N] weight): an instruction covers 1024/BN k rows; lane l -> row b*(1024/BN) + l/(BN/16),
     // LDS chunk l%(BN/16), global chunk (l%(BN/16)) ^ h(row)
-    auto voff_kn = [&](int b) {
+    auto voff_kn = [&](int b, uint32_t k0) {
         constexpr int CPR = BN / 16;
         const int row = b * (1024 / BN) + lane / CPR;
-        return (uint32_t)row * ldb + 16u * (uint32_t)((lane % CPR) ^ md::hkn<BN>(row));
+        return !RAG || k0 + (uint32_t)row < K ? (uint32_t)row * ldb + 16u * (uint32_t)((lane % CPR) ^ md::hkn<BN>(row)) : kOutside;
     };
-    const int nk = (int)(p.K / md::KS / (SPLIT ? nsplit : 1));  // stages of this workgroup's K range
+    // stages of this workgroup's K range (a split only where K is whole stages per split)
+    const int nk = RAG ? (int)((p.K + md::KS - 1) / md::KS) : (int)(p.K / md::KS / (SPLIT ? nsplit : 1));
     const uint32_t kbeg = (uint32_t)(split * nk * md::KS);
     const bool hi = wave < C::DMA % NW;  // this wave issues PW_HI instructions per stage
     auto issue = [&](int s) {  // stage s into buffer s % NST: instructions wave, wave+NW, ...
@@ -1222,12 +1256,12 @@ __global__ __launch_bounds__(64 * NW + (PD > 0 ? 64 : 0)) void qmm_mid(QmmArgs p
             const int q = wave + NW * u;
             if (q >= C::DMA) break;
             if (q < C::A_DMA) {
-                dma16(rsA, lds + q * 1024, voff_rk(q, lda), k0);
+                dma16(rsA, lds + q * 1024, voff_rk(q, lda, k0), k0);
             } else {
                 const int b = q - C::A_DMA;
                 if constexpr (B_NZ) dma16(rsB, lds + C::A_BYTES + b * 1024, voff_nz(b, k0), 0u);
-                else if constexpr (B_KN) dma16(rsB, lds + C::A_BYTES + b * 1024, voff_kn(b), k0 * ldb);
-                else dma16(rsB, lds + C::A_BYTES + b * 1024, voff_rk(b, ldb), k0);
+                else if constexpr (B_KN) dma16(rsB, lds + C::A_BYTES + b * 1024, voff_kn(b, k0), k0 * ldb);
+                else dma16(rsB, lds + C::A_BYTES + b * 1024, voff_rk(b, ldb, k0), k0);
             }
         }
     };
@@ -1254,10 +1288,10 @@ __global__ __launch_bounds__(64 * NW + (PD > 0 ? 64 : 0)) void qmm_mid(QmmArgs p
         const uint32_t lds = sbase + (uint32_t)(NST * C::STAGE);
         const uint32_t k0 = kbeg + (uint32_t)s * md::KS;
         if (pf_a)
-            for (int q = 0; q < C::A_DMA; ++q) dma16(rsA, lds, voff_rk(q, lda), k0);
+            for (int q = 0; q < C::A_DMA; ++q) dma16(rsA, lds, voff_rk(q, lda, k0), k0);
         for (int b = tm; b < BN / 4; b += tiles_m) {
-            if constexpr (B_KN) dma16(rsB, lds, voff_kn(b), k0 * ldb);
-            else dma16(rsB, lds, voff_rk(b, ldb), k0);
+            if constexpr (B_KN) dma16(rsB, lds, voff_kn(b, k0), k0 * ldb);
+            else dma16(rsB, lds, voff_rk(b, ldb, k0), k0);
         }
     };
     if (pf_wave) {
@@ -1333,7 +1367,7 @@ __global__ __launch_bounds__(64 * NW + (PD > 0 ? 64 : 0)) void qmm_mid(QmmArgs p
     // int32 sum of the four K partials, then (this split's share of) the epilogue
     static_assert(BM * BN / 8 <= NT, "one group of 8 outputs per thread");
     const int row = tid / (BN / 8), c8 = 8 * (tid % (BN / 8));
-    const bool has = !pf_wave && tid < BM * BN / 8 && row < rows;
+    const bool has = !pf_wave && tid < BM * BN / 8 && row < rows && (!RAG || n0 + c8 < p.N);
     uint32_t s8[8];
 #pragma unroll
     for (int t = 0; t < 8; ++t) s8[t] = 0u;
@@ -1582,6 +1616,7 @@ __global__ __launch_bounds__(kThreads) void qmm_reduce_tiled(QmmArgs p, int tile
         const int tm = first_m + (bid % per_group) % gm, tn = (bid % per_group) / gm;
         const int64_t m = (int64_t)tm * BM + (wave >> 1) * (BM / 4) + 16 * (f >> 3) + 4 * (lane >> 4);
         const int64_t n = (int64_t)tn * 256 + (wave & 1) * 128 + 16 * (f & 7) + (lane & 15);
+        if (n >= p.N) continue;  // the last column tile of a ragged N
         if (!half) {
             uint32_t s[4] = {0u, 0u, 0u, 0u};
             for (int k = 0; k < NS; ++k) {
@@ -1670,9 +1705,16 @@ bool big_nk_full(const QmmArgs& p, int nsplit) {
 // ranges of whole 4-stage rings, 16-byte aligned rows, and every operand range of a tile addressable by a
 // 32-bit buffer offset.
 bool big_dma_ok(const QmmArgs& p, bool b_kn, int nsplit) {
-    return plan_override().qmm_dma && big_nk_full(p, nsplit) && (p.K / nsplit) % (dm::BK * dm::NST) == 0 &&
-           p.lda % 16 == 0 && (uintptr_t)p.a % 16 == 0 && (uintptr_t)p.b % 16 == 0 &&
-           (b_kn ? (p.sbk % 16 == 0 && (uint64_t)p.K * (uint64_t)p.sbk < (1ull << 32)) : (p.sbn % 16 == 0));
+    (void)nsplit;
+    return plan_override().qmm_dma && p.K > 0 && p.K % 16 == 0 && p.lda < (1 << 24) && p.sbk < (1 << 24) &&
+           p.sbn < (1 << 24) && p.lda % 16 == 0 && (uintptr_t)p.a % 16 == 0 && (uintptr_t)p.b % 16 == 0 &&
+           (uintptr_t)p.epi.out % 16 == 0 && p.epi.ldo % 8 == 0 &&
+           (b_kn ? (p.N % 16 == 0 && p.sbk % 16 == 0 && (uint64_t)p.K * (uint64_t)p.sbk < (1ull << 32))
+                 : (p.N % 8 == 0 && p.sbn % 16 == 0));
+}
+
+bool dma_ragged(const QmmArgs& p, int nsplit) {
+    return p.N % dm::BN != 0 || p.K % ((int64_t)nsplit * dm::BK * dm::NST) != 0;
 }
 
 // qmm_dma's round length for walking K backwards in every other round: one workgroup per CU (INT_MAX: never)
@@ -1689,8 +1731,9 @@ hipError_t launch_big(const QmmArgs& p, bool b_kn, int tiles_m, int tiles_n, int
     const bool dma = big_dma_ok(p, b_kn, nsplit);
     if (nsplit > 1 && !full && !dma) return hipErrorInvalidValue;  // not planned (launch_quant_matmul unsplits)
     if (dma) {
-        if (b_kn) qmm_dma<kLayKN, OUT><<<grid, dim3(dm::NT), 0, stream>>>(p, tiles_m, tiles_n, nsplit, partial, dma_rev_from());
-        else qmm_dma<kLayNK, OUT><<<grid, dim3(dm::NT), 0, stream>>>(p, tiles_m, tiles_n, nsplit, partial, dma_rev_from());
+        const auto k = dma_ragged(p, nsplit) ? (b_kn ? qmm_dma<kLayKN, OUT, 256, true> : qmm_dma<kLayNK, OUT, 256, true>)
+                                             : (b_kn ? qmm_dma<kLayKN, OUT> : qmm_dma<kLayNK, OUT>);
+        k<<<grid, dim3(dm::NT), 0, stream>>>(p, tiles_m, tiles_n, nsplit, partial, dma_rev_from());
     } else if (full) {
         if (b_kn) qmm_big<true, OUT, 8, true><<<grid, dim3(512), 0, stream>>>(p, tiles_m, tiles_n, nsplit, partial);
         else qmm_big<false, OUT, 8, true><<<grid, dim3(512), 0, stream>>>(p, tiles_m, tiles_n, nsplit, partial);
@@ -1714,12 +1757,20 @@ struct BigPlan {
     bool ok = false;
     int tiles_m = 0, tiles_n = 0, nsplit = 1;
     int bm = 256;
+    bool ragged = false;  // a K split only the direct-to-LDS kernel can run (a ragged N, or uneven in K)
 };
 
 // the power-of-two K split that brings `tiles` to about 192 workgroups (each split at least 512 deep)
 int big_splits(int64_t tiles, int64_t K) {
     int ns = 1;
     while (tiles * ns < 192 && ns < 16 && K % ((int64_t)ns * 2 * big::BK) == 0 && K / (ns * 2) >= 512) ns *= 2;
+    return ns;
+}
+
+// the same for a ragged N or a K with no even split: ranges of whole 256-K rings, the last one shorter
+int big_splits_ragged(int64_t tiles, int64_t K) {
+    int ns = 1;
+    while (tiles * ns < 192 && ns < 16 && K / (ns * 2) >= 512 && (2 * ns - 1) * dma_k_len(K, 2 * ns) < K) ns *= 2;
     return ns;
 }
 
@@ -1733,18 +1784,22 @@ BigPlan big_plan(int64_t M, int64_t N, int64_t K, bool allow128 = true) {
         b.ok = true;
         return b;
     }
-    // a split needs whole tiles along N and K; a ragged M only runs split on the direct-to-LDS kernel
-    if (N % big::BN != 0 || K % big::BK != 0) return b;
-    const int ns = big_splits(tm * tn, K);
-    if (ns == 1 || tm * tn * ns < 64 || (int64_t)ns * M * N * 4 > ((int64_t)512 << 20)) return b;
+    // A split of the register-staged kernel needs whole tiles along N and K.  The direct-to-LDS kernel also splits
+    // a ragged N, a K of no even split (11008 = 43 x 256, 13696, 5504) and a ragged M; those shapes ran unsplit
+    // 128 x 128 tiles of the generic tiled kernel (M = 250, K = 13696, N = 5120: 240 us, now 47).
+    int ns = N % big::BN == 0 && K % big::BK == 0 ? big_splits(tm * tn, K) : 1;
+    const bool even = ns > 1;
+    if (!even && N % 8 == 0 && K % 16 == 0) ns = big_splits_ragged(tm * tn, K);
+    b.ragged = !even;
+    if (ns == 1 || (even && tm * tn * ns < 64) || (int64_t)ns * M * N * 4 > ((int64_t)512 << 20)) return b;
     b.nsplit = ns;
     b.ok = true;
     // 128-row tiles run only as K splits (their kernel writes int32 partials): where the 128-row tiles alone
     // already fill the CUs (ns2 == 1) the 256-row split stays
     const int64_t tm2 = (M + 127) / 128;
-    const int ns2 = big_splits(tm2 * tn, K);
-    if (allow128 && plan_override().qmm_bm128 && ns2 > 1 && ns2 < ns && tm2 * tn * ns2 >= 64 &&
-        K % ((int64_t)ns2 * dm::BK * dm::NST) == 0) {
+    const int ns2 = even ? big_splits(tm2 * tn, K) : big_splits_ragged(tm2 * tn, K);
+    if (allow128 && plan_override().qmm_bm128 && ns2 > 1 && ns2 < ns && ns2 <= 8 &&
+        (!even || (tm2 * tn * ns2 >= 64 && K % ((int64_t)ns2 * dm::BK * dm::NST) == 0))) {
         b.bm = 128;
         b.tiles_m = (int)tm2;
         b.nsplit = ns2;
@@ -1755,13 +1810,15 @@ BigPlan big_plan(int64_t M, int64_t N, int64_t K, bool allow128 = true) {
 // [split-K counters][partials]: int32 [nsplit][M][N], or for 128-row tiles [nsplit][tiles][128 x 256]
 size_t big_split_workspace(const BigPlan& b, int64_t M, int64_t N) {
     const size_t rows = b.bm == 128 ? (size_t)b.tiles_m * 128 : (size_t)M;
-    return QK_SPLIT_COUNTER_BYTES + (size_t)b.nsplit * rows * (size_t)N * sizeof(int32_t);
+    const size_t cols = b.bm == 128 ? (size_t)b.tiles_n * 256 : (size_t)N;
+    return QK_SPLIT_COUNTER_BYTES + (size_t)b.nsplit * rows * cols * sizeof(int32_t);
 }
 
 template <int BL>
 hipError_t launch_split128(const QmmArgs& p, const BigPlan& b, int32_t* partial, hipStream_t stream) {
     const dim3 sgrid((uint32_t)((int64_t)b.tiles_m * b.tiles_n * b.nsplit)), sblock(dm::NT);
-    qmm_dma<BL, QK_I32, 128><<<sgrid, sblock, 0, stream>>>(p, b.tiles_m, b.tiles_n, b.nsplit, partial, dma_rev_from());
+    const auto k = dma_ragged(p, b.nsplit) ? qmm_dma<BL, QK_I32, 128, true> : qmm_dma<BL, QK_I32, 128>;
+    k<<<sgrid, sblock, 0, stream>>>(p, b.tiles_m, b.tiles_n, b.nsplit, partial, dma_rev_from());
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     int64_t blocks = ((int64_t)b.tiles_m * b.tiles_n * 8 * 16 * 64 + kThreads - 1) / kThreads;
@@ -1803,6 +1860,14 @@ SkinnyPlan skinny_plan(int64_t M, int64_t N, int64_t K) {
         return K % (ns * sk::BK) == 0 && ns * M * 4 <= K && K / ns >= 256;
     };
     while (base * s.nsplit * 2 <= target && fits((int64_t)s.nsplit * 2)) s.nsplit *= 2;
+    // a K that the doubling cannot split evenly (11008 = 86 stages, 13696 = 107): the largest count of splits of
+    // whole stages, the last one shorter (M = 20, K = 11008, N = 4096: 41 -> 20 us)
+    if (base * s.nsplit * 2 <= target && K % ((int64_t)s.nsplit * 2 * sk::BK) != 0)
+        for (int64_t ns = target / base; ns > s.nsplit; --ns)
+            if (ns * M * 4 <= K && K / ns >= 256 && (ns - 1) * sk::sk_k_len(K, ns) < K) {
+                s.nsplit = (int)ns;
+                break;
+            }
     // debug override: a power of two within the same bounds as the planned count
     if (const int v = plan_override().skinny_splits) {
         if (v == 1 || fits(v)) s.nsplit = v;
@@ -1855,7 +1920,7 @@ hipError_t launch_skinny(const QmmArgs& p, const SkinnyPlan& s, int32_t* partial
 }  // namespace
 
 // Mid-M shapes (M <= 128, or M <= 256 with N <= 8192 -- beyond that the 256x256 tiles move fewer bytes
-// per CU; N % 64 == 0, K % 256 == 0): qmm_mid, no workspace.  Column blocks of 128 for a [K,N]
+// per CU; N % 64 == 0 on [K,N], N % 8 == 0 on the other layouts; K % 16 == 0): qmm_mid, no workspace.  Column blocks of 128 for a [K,N]
 // weight whose N allows it (whole-line k rows), else 64; the row block (64, 32 or 16; 32 at most with
 // 128 columns) that moves the fewest operand bytes per CU.  A [K,N] weight with M <= 32 keeps the split
 // stream (measured faster there), so for M <= 32 the workspace query still reports the split stream's
@@ -1872,11 +1937,13 @@ struct MidPlan {
 MidPlan mid_plan(int64_t M, int64_t N, int64_t K, bool b_kn) {
     MidPlan m;
     if (!plan_override().qmm_mid) return m;  // debug override: the split stream / tiled kernels instead
-    if (M <= 0 || M > 256 || (M > 128 && N > 8192) || N <= 0 || N % 64 != 0 || K <= 0 || K % md::KS != 0)
+    // any K of whole 16-byte chunks (the last stage may be partly past it); a ragged last column block except on
+    // [K,N] rows
+    if (M <= 0 || M > 256 || (M > 128 && N > 8192) || N <= 0 || N % (b_kn ? 64 : 8) != 0 || K <= 0 || K % 16 != 0)
         return m;
     const PlanOverride& ov = plan_override();  // debug override: a row block, column block and / or split
     const int bn = (b_kn && N % 128 == 0 && ov.mid_bn != 64) ? 128 : 64;
-    const int64_t tn = N / bn;
+    const int64_t tn = (N + bn - 1) / bn;
     if (tn * ((M + 15) / 16) >= ((int64_t)1 << 30)) return m;
     // the row block (and, with 128 columns, K split) with the fewest bytes per CU: rounds of workgroups over
     // the 256 CUs times each workgroup's (BM + BN) * K / nsplit operand bytes, plus a split's partial tile
@@ -1928,25 +1995,28 @@ size_t mid_workspace(const MidPlan& m) {
 //            weight at its HBM rate;
 //   split:   the larger of its fill time (the M rows of A: rows past M read as zeros without a fetch) and its
 //            HBM time (the weight and the partials written), plus the reduce of the partials.
-// The split count with the lowest estimate is taken when it is below 0.9 of qmm_mid's.  The sums are exact, so
-// the bits equal qmm_mid's.  Returns the split count, or 0 for qmm_mid.
+// The split count with the lowest estimate is taken when it is below 0.9 of qmm_mid's; 0.82 on an NZ weight of at
+// most two rounds of qmm_mid's workgroups, where its estimate is closest and the split's runs a tenth low
+// (K = 11008, N = 4096, M = 70-128: qmm_mid 22-23 us, 8 splits 24.4-25.8; K = 8192, N = 3584: 17.1-17.7 against
+// 19.8-20.4; K = 13696, N = 5120, M = 100: 37.0 against 31.8; four rounds, K = 4096, N = 28672, M = 90: 52.1
+// against 40.5).  The sums are exact, so the bits equal qmm_mid's.  Returns the split count, or 0 for qmm_mid.
 constexpr double kMidHbmKn = 3.1e6, kMidHbmNz = 4.6e6;  // qmm_mid's weight read rate, bytes per us
 
 int small_split(int64_t M, int64_t N, int64_t K, const MidPlan& mp, double mid_hbm = kMidHbmKn) {
     const PlanOverride& ov = plan_override();  // debug override: qmm_small=0 never, =<n> that split count
-    if (ov.qmm_small == 0 || mp.bm == 0 || M <= 32 || M > 128 || N % 256 != 0 || K <= 0) return 0;
+    if (ov.qmm_small == 0 || mp.bm == 0 || M <= 32 || M > 128 || N % 16 != 0 || K <= 0) return 0;
     auto rounds = [](int64_t wgs) { return (double)((wgs + 255) / 256); };
     constexpr double kFill = 45e3, kHbm = 5e6, kReduce = 4e6, kReduceFixed = 3.0;  // bytes per us; us
     const double w_bytes = (double)K * (double)N;
     const double t_mid_fill = rounds((int64_t)mp.tiles * mp.nsplit) * (mp.bm + mp.bn) * (double)(K / mp.nsplit) / kFill;
     const double t_mid = t_mid_fill > w_bytes / mid_hbm ? t_mid_fill : w_bytes / mid_hbm;
     int best = 0;
-    double t_best = 0.9 * t_mid;
+    double t_best = (mid_hbm == kMidHbmNz && mp.tiles <= 512 ? 0.82 : 0.9) * t_mid;
     for (int ns : {2, 4, 8}) {
         if (ov.qmm_small > 0 && ns != ov.qmm_small) continue;
-        if (K % ((int64_t)ns * dm::BK * dm::NST) != 0) continue;
+        if (K / ns < 256 || (ns - 1) * dma_k_len(K, ns) >= K) continue;
         const double part = (double)ns * 128.0 * (double)N * 4.0;
-        const double t_fill = rounds(N / 256 * ns) * (double)(M + 256) * (double)(K / ns) / kFill;
+        const double t_fill = rounds((N + 255) / 256 * ns) * (double)(M + 256) * (double)dma_k_len(K, ns) / kFill;
         const double t_hbm = (w_bytes + part) / kHbm;
         const double t = (t_fill > t_hbm ? t_fill : t_hbm) + part / kReduce + kReduceFixed;
         if (ov.qmm_small > 0 || t < t_best) {
@@ -1962,7 +2032,7 @@ BigPlan small_split_plan(int64_t M, int64_t N, int ns) {
     b.ok = true;
     b.bm = 128;
     b.tiles_m = (int)((M + 127) / 128);
-    b.tiles_n = (int)(N / 256);
+    b.tiles_n = (int)((N + 255) / 256);
     b.nsplit = ns;
     return b;
 }
@@ -1979,6 +2049,8 @@ hipError_t launch_mid_o(const QmmArgs& p, const MidPlan& mp, int32_t* partial, u
                                                                                 ctr, next_split_tag());
         else
             return hipErrorInvalidValue;
+    } else if (p.N % BN != 0 || p.K % md::KS != 0) {
+        qmm_mid<BL, BM, BN, NW, PD, OUT, false, true><<<grid, block, 0, stream>>>(p, mp.tiles_m, 1, nullptr, nullptr, 0);
     } else {
         qmm_mid<BL, BM, BN, NW, PD, OUT, false><<<grid, block, 0, stream>>>(p, mp.tiles_m, 1, nullptr, nullptr, 0);
     }
@@ -2022,26 +2094,28 @@ hipError_t launch_qmm_fallback(const QmmArgs& p, bool a_ok, bool b_kn, bool b_nk
 
 // A split workspace is [split-K counters][int32 partials [nsplit][M][N]].
 size_t quant_matmul_workspace(int64_t M, int64_t N, int64_t K) {
-    if (mid_plan(M, N, K, false).bm != 0 && M > 32) {  // eligibility does not depend on the layout; the
-        const MidPlan mk = mid_plan(M, N, K, true);     // [K,N] plan's splits need a workspace
-        size_t need = mid_workspace(mk);
+    size_t need = 0;
+    if (mid_plan(M, N, K, true).bm != 0 && M > 32) {  // where [K,N] runs qmm_mid, the other layouts do too; the
+        const MidPlan mk = mid_plan(M, N, K, true);    // [K,N] plan's splits need a workspace
+        need = mid_workspace(mk);
         if (const int ns = small_split(M, N, K, mk)) {
             const size_t alt = big_split_workspace(small_split_plan(M, N, ns), M, N);
             if (alt > need) need = alt;
         }
-        return need;
+        if (K % md::KS == 0) return need;  // else operands qmm_mid cannot take go on to the plans below
     }
     const SkinnyPlan s = skinny_plan(M, N, K);
-    if (s.mt != 0)
-        return s.nsplit == 1 ? 0 : QK_SPLIT_COUNTER_BYTES + (size_t)s.nsplit * (size_t)M * (size_t)N * sizeof(int32_t);
-    const BigPlan b = big_plan(M, N, K);
-    if (!b.ok || b.nsplit == 1) return 0;
-    // a 128-row split plan falls back to the 256-row one where its kernel does not apply: room for either
-    const size_t need = big_split_workspace(b, M, N);
-    if (b.bm == 128) {
-        const size_t alt = big_split_workspace(big_plan(M, N, K, false), M, N);
+    if (s.mt != 0) {
+        const size_t alt =
+            s.nsplit == 1 ? 0 : QK_SPLIT_COUNTER_BYTES + (size_t)s.nsplit * (size_t)M * (size_t)N * sizeof(int32_t);
         return need > alt ? need : alt;
     }
+    const BigPlan b = big_plan(M, N, K);
+    if (!b.ok || b.nsplit == 1) return need;
+    size_t alt = big_split_workspace(b, M, N);
+    if (alt > need) need = alt;
+    // a 128-row split plan falls back to the 256-row one where its kernel does not apply: room for either
+    if (b.bm == 128 && (alt = big_split_workspace(big_plan(M, N, K, false), M, N)) > need) need = alt;
     return need;
 }
 
@@ -2054,7 +2128,8 @@ hipError_t launch_quant_matmul(const QmmArgs& p, void* workspace, size_t ws_byte
     char* ws = static_cast<char*>(workspace);
     int32_t* partial = ws ? reinterpret_cast<int32_t*>(ws + QK_SPLIT_COUNTER_BYTES) : nullptr;
     MidPlan mp = mid_plan(p.M, p.N, p.K, b_kn16);
-    if (mp.bm != 0 && (p.M > 32 || !b_kn16)) {
+    const SkinnyPlan sp = skinny_plan(p.M, p.N, p.K);
+    if (mp.bm != 0 && (p.M > 32 || !b_kn16 || sp.mt == 0)) {
         if (b_kn16) {  // wide or deep [K,N] weights: 128-row K splits where the cost model favours them
             if (const int ns = small_split(p.M, p.N, p.K, mp)) {
                 const BigPlan sb = small_split_plan(p.M, p.N, ns);
@@ -2075,9 +2150,8 @@ hipError_t launch_quant_matmul(const QmmArgs& p, void* workspace, size_t ws_byte
                                 : (b_nk && (uint64_t)mp.bn * (uint64_t)p.sbn < (1ull << 32)));
         uint64_t* ctr = mp.nsplit > 1 ? reinterpret_cast<uint64_t*>(ws) : nullptr;
         if (ok) return b_kn16 ? launch_mid<kLayKN>(p, mp, partial, ctr, stream) : launch_mid<kLayNK>(p, mp, partial, ctr, stream);
-        return launch_qmm_fallback(p, a_ok, b_kn, b_nk, stream);
+        if (p.N % 64 == 0 && p.K % md::KS == 0) return launch_qmm_fallback(p, a_ok, b_kn, b_nk, stream);
     }
-    const SkinnyPlan sp = skinny_plan(p.M, p.N, p.K);
     if (sp.mt != 0 && a_ok && (b_nk || b_kn16)) {
         const size_t need = sp.nsplit > 1 ? QK_SPLIT_COUNTER_BYTES + (size_t)sp.nsplit * p.M * p.N * sizeof(int32_t) : 0;
         if (need && (!workspace || ws_bytes < need)) return hipErrorInvalidValue;
@@ -2092,6 +2166,8 @@ hipError_t launch_quant_matmul(const QmmArgs& p, void* workspace, size_t ws_byte
             return b_kn ? launch_split128<kLayKN>(p, bp, partial, stream) : launch_split128<kLayNK>(p, bp, partial, stream);
         bp = big_plan(p.M, p.N, p.K, false);
     }
+    // a ragged split runs only on the direct-to-LDS kernel; otherwise the tiled kernels take the shape
+    if (big_ok && bp.ragged && bp.nsplit > 1 && !big_dma_ok(p, b_kn, bp.nsplit)) big_ok = false;
     // a split of a ragged M runs only on the direct-to-LDS kernel; otherwise the register-staged kernel runs
     // the shape unsplit (the planned workspace is then unused)
     if (big_ok && bp.nsplit > 1 && p.M % big::BM != 0 && !big_dma_ok(p, b_kn, bp.nsplit)) bp.nsplit = 1;
@@ -2165,16 +2241,15 @@ hipError_t launch_nzd(const QmmArgs& p, const NzdPlan& z, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// qmm_dma on NZ blocks: whole 256-column tiles (any M) and K ranges of whole four-stage rings
-bool nz_dma_ok(const BigPlan& b, int64_t M, int64_t N, int64_t K) {
-    (void)M;
-    return plan_override().qmm_dma && b.ok && N % dm::BN == 0 && K % ((int64_t)b.nsplit * dm::BK * dm::NST) == 0;
-}
+// qmm_dma on NZ blocks: every shape with a plan (any M, N and K; the last column tile and the last K range of an
+// NZ weight may be ragged)
+bool nz_dma_ok(const BigPlan& b) { return plan_override().qmm_dma && b.ok; }
 
 template <int OUT>
 hipError_t launch_dma_nz(const QmmArgs& p, const BigPlan& b, int32_t* partial, hipStream_t stream) {
     if (b.bm != 256) return hipErrorInvalidValue;  // 256-row tiles: tiles_m counts them
-    qmm_dma<kLayNZ, OUT><<<dim3((uint32_t)(b.tiles_m * b.tiles_n * b.nsplit)), dim3(dm::NT), 0, stream>>>(
+    const auto k = dma_ragged(p, b.nsplit) ? qmm_dma<kLayNZ, OUT, 256, true> : qmm_dma<kLayNZ, OUT>;
+    k<<<dim3((uint32_t)(b.tiles_m * b.tiles_n * b.nsplit)), dim3(dm::NT), 0, stream>>>(
         p, b.tiles_m, b.tiles_n, b.nsplit, partial, dma_rev_from());
     return hipGetLastError();
 }
@@ -2191,7 +2266,7 @@ size_t quant_matmul_nz_workspace(int64_t M, int64_t N, int64_t K) {
         return ns ? big_split_workspace(small_split_plan(M, N, ns), M, N) : 0;
     }
     const BigPlan b = big_plan(M, N, K);
-    if (nz_dma_ok(b, M, N, K)) return b.nsplit > 1 ? big_split_workspace(b, M, N) : 0;
+    if (nz_dma_ok(b)) return b.nsplit > 1 ? big_split_workspace(b, M, N) : 0;
     return round_up256((size_t)K * (size_t)N) + quant_matmul_workspace(M, N, K);
 }
 
@@ -2215,7 +2290,7 @@ hipError_t launch_quant_matmul_nz(const QmmArgs& p, void* workspace, size_t ws_b
         return launch_mid<kLayNZ>(p, mp, nullptr, nullptr, stream);
     }
     const BigPlan b = big_plan(p.M, p.N, p.K);
-    if (nz_dma_ok(b, p.M, p.N, p.K)) {
+    if (nz_dma_ok(b)) {
         if (b.nsplit == 1) {
             switch (p.epi.out_dtype) {
             case QK_BF16: return launch_dma_nz<QK_BF16>(p, b, nullptr, stream);
