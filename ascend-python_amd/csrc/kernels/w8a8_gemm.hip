@@ -1786,7 +1786,7 @@ BigPlan big_plan(int64_t M, int64_t N, int64_t K, bool allow128 = true) {
     }
     // A split of the register-staged kernel needs whole tiles along N and K.  The direct-to-LDS kernel also splits
     // a ragged N, a K of no even split (11008 = 43 x 256, 13696, 5504) and a ragged M; those shapes ran unsplit
-    // 128 x 128 tiles of the generic tiled kernel (M = 250, K = 13696, N = 5120: 240 us, now 47).
+    // 128 x 128 tiles of the generic tiled kernel (M = 300, K = 13696, N = 5120, quantization included: 261 us, now 47).
     int ns = N % big::BN == 0 && K % big::BK == 0 ? big_splits(tm * tn, K) : 1;
     const bool even = ns > 1;
     if (!even && N % 8 == 0 && K % 16 == 0) ns = big_splits_ragged(tm * tn, K);

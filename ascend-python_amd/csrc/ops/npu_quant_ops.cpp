@@ -874,6 +874,13 @@ std::tuple<at::Tensor, at::Tensor> npu_swiglu_dynamic_quant_meta(const at::Tenso
 }
 
 // ---------------------------------------------------------------- fused gate-up + SwiGLU (quantized MLP block)
+// Up to this many rows the gate-up product runs the small-M GEMMs and a SwiGLU pass over its [M, 2I] output instead
+// of the fused kernel, whose 256-row tiles then mostly multiply padding and, one tile row high, occupy I / 128 CUs
+// (same bits; us, fused against chain with the quantization, NZ / [K,N] weight: K = 4096, I = 14336 M = 1 44.0 /
+// 54.5 against 24.9 / 28.9, M = 64 45.7 / 57.2 against 35.5 / 48.4, M = 128 47.0 / 60.3 against 42.8 / 44.9; K =
+// 2048, I = 5504 M = 16 29.1 / 31.2 against 12.7 / 16.8.  At M = 160 the two are level on NZ (48.3 / 49.5), and at
+// I = 11008 the fused kernel is ahead (45.6 / 52.1)).
+constexpr int64_t kSwigluChainRows = 128;
 // h = npu_swiglu(npu_quant_matmul(x1, x2, scale, pertoken_scale=..., output_dtype=...)) with x2 [K, 2I] (row-major
 // or the int8 NZ weight) in one GEMM whose epilogue applies the SwiGLU: bit-identical to that chain, which it
 // runs instead where the fused kernel does not take the shape (qk_quant_matmul_swiglu: QK_ERR_UNSUPPORTED).
@@ -903,6 +910,9 @@ std::vector<int64_t> swiglu_matmul_check(const at::Tensor& x1, const at::Tensor&
     return shape;
 }
 
+// npu_quant_matmul takes 2 to 6 dims; the fused kernels any x1 of at least 2
+bool swiglu_chain(const at::Tensor& x1) { return leading_rows(x1) <= kSwigluChainRows && x1.dim() <= 6; }
+
 at::Tensor npu_quant_matmul_swiglu(const at::Tensor& x1_in, const at::Tensor& x2_in, const at::Tensor& scale_in,
                                    const std::optional<at::Tensor>& pertoken_scale,
                                    std::optional<at::ScalarType> output_dtype) {
@@ -915,7 +925,7 @@ at::Tensor npu_quant_matmul_swiglu(const at::Tensor& x1_in, const at::Tensor& x2
     const bool nz = is_w8_nz(x2_in);
     auto x1 = x1_in.contiguous();
     const bool kn = !nz && x2_in.stride(1) == 1 && x2_in.stride(0) >= 2 * I;
-    if (nz || kn) {
+    if ((nz || kn) && !swiglu_chain(x1)) {
         auto scale = scale_in.scalar_type() == at::kFloat ? scale_in.contiguous() : scale_in.to(at::kFloat);
         at::Tensor pt;
         if (pertoken_scale.has_value()) pt = pertoken_scale->contiguous();
@@ -928,14 +938,14 @@ at::Tensor npu_quant_matmul_swiglu(const at::Tensor& x1_in, const at::Tensor& x2
             return out;
         }
     }
-    // the shapes and layouts the fused kernel does not take: the unfused chain
+    // few rows, and the shapes and layouts the fused kernel does not take: the unfused chain
     auto h2 = npu_quant_matmul(x1_in, x2_in, scale_in, std::nullopt, pertoken_scale, std::nullopt, out_type);
     return npu_swiglu(h2, -1);
 }
 
 // (q, q_scale) = npu_dynamic_quant(npu_quant_matmul_swiglu(...)) bit for bit: h and the GEMM's per-row partial
-// absmax in a workspace, then one elementwise quantizing pass (qk_quant_matmul_swiglu_quant); the chain where
-// the fused kernels do not take the shape.
+// absmax in a workspace, then one elementwise quantizing pass (qk_quant_matmul_swiglu_quant); the chain for few
+// rows and where the fused kernels do not take the shape.
 std::tuple<at::Tensor, at::Tensor> npu_quant_matmul_swiglu_quant(const at::Tensor& x1_in, const at::Tensor& x2_in,
                                                                  const at::Tensor& scale_in,
                                                                  const std::optional<at::Tensor>& pertoken_scale,
@@ -950,7 +960,7 @@ std::tuple<at::Tensor, at::Tensor> npu_quant_matmul_swiglu_quant(const at::Tenso
     const bool nz = is_w8_nz(x2_in);
     auto x1 = x1_in.contiguous();
     const bool kn = !nz && x2_in.stride(1) == 1 && x2_in.stride(0) >= 2 * I;
-    if (nz || kn) {
+    if ((nz || kn) && !swiglu_chain(x1)) {
         auto scale = scale_in.scalar_type() == at::kFloat ? scale_in.contiguous() : scale_in.to(at::kFloat);
         at::Tensor pt;
         if (pertoken_scale.has_value()) pt = pertoken_scale->contiguous();
@@ -968,7 +978,9 @@ std::tuple<at::Tensor, at::Tensor> npu_quant_matmul_swiglu_quant(const at::Tenso
             return {q, qs};
         }
     }
-    return npu_dynamic_quant(npu_quant_matmul_swiglu(x1_in, x2_in, scale_in, pertoken_scale, h_type), std::nullopt);
+    // the chain, SwiGLU and quantization in one pass ([N,K] weights, M = 16: 37.5 -> 34.9 us)
+    return npu_swiglu_dynamic_quant(
+        npu_quant_matmul(x1_in, x2_in, scale_in, std::nullopt, pertoken_scale, std::nullopt, h_type), -1);
 }
 
 std::tuple<at::Tensor, at::Tensor> npu_quant_matmul_swiglu_quant_meta(const at::Tensor& x1, const at::Tensor& x2,
