@@ -368,7 +368,10 @@ __global__ __launch_bounds__(kThreads) void w4_decode(WqbmmArgs p, float* __rest
 // 8- or 16-byte load per row) and their 4*LW bytes (MFMA tiles, columns
 // 4*LW*c + t), and the operands are the exact 16-bit values of the bytes (no
 // magic offset: BASE = 0).
-template <int DT, int WPL, int NWAVE, int NKB, int PF, int PIECE_KB, bool HAS_OFF, bool FINAL, bool W8>
+// RAG: the last split reaches past K (K is whole 32-row blocks): the lanes of a block past K load from outside the
+// resources (zeros, no memory access) and a piece past K folds with scale and offset 0.  An instance of its own: the
+// selects cost the even shapes 2-3 us (K = 4096, N = 4096, M = 1: 7.8 -> 10.5).
+template <int DT, int WPL, int NWAVE, int NKB, int PF, int PIECE_KB, bool HAS_OFF, bool FINAL, bool W8, bool RAG = false>
 __global__ __launch_bounds__(64 * NWAVE) void w4_stream(WqbmmArgs p, float* __restrict__ partial, int nstrip,
                                                         int nsplit, uint64_t* __restrict__ ctr, uint64_t tag) {
     typedef Mfma<DT> MM;
@@ -409,11 +412,9 @@ __global__ __launch_bounds__(64 * NWAVE) void w4_stream(WqbmmArgs p, float* __re
     const int k_wave = split * (KW * NKB * 32) + kw * (NKB * 32);
 
     // buffer resources over this wave's rows: lane offsets in VGPRs, row
-    // offsets in SGPRs (no per-load address arithmetic).  The last split may
-    // reach past K (K is whole 32-row blocks): the lanes of a block past K
-    // load from outside the resources, zeros without a memory access.
+    // offsets in SGPRs (no per-load address arithmetic)
     const uint32_t rowbytes = (uint32_t)NW * 4u;
-    const int k_left = K - k_wave < NKB * 32 ? (K - k_wave > 0 ? K - k_wave : 0) : NKB * 32;
+    const int k_left = !RAG ? NKB * 32 : K - k_wave < NKB * 32 ? (K - k_wave > 0 ? K - k_wave : 0) : NKB * 32;
     const __amdgpu_buffer_rsrc_t wr =
         make_rsrc(static_cast<const char*>(p.w) + (size_t)(uint32_t)k_wave * rowbytes, (uint32_t)k_left * rowbytes);
     const uint32_t w_lane = (uint32_t)(8 * kg) * rowbytes + (uint32_t)wc * 4u;
@@ -432,7 +433,7 @@ __global__ __launch_bounds__(64 * NWAVE) void w4_stream(WqbmmArgs p, float* __re
     SV sv[NPIECE][SVN], ov[NPIECE][SVN];
 #pragma unroll
     for (int pc = 0; pc < NPIECE; ++pc) {
-        const bool in = pc * PIECE_KB * 32 < k_left;  // a piece past K: scale and offset 0, so its fold adds 0
+        const bool in = !RAG || pc * PIECE_KB * 32 < k_left;
         const uint32_t g = in ? (uint32_t)(k_wave + pc * PIECE_KB * 32) / (uint32_t)G : 0u;
         const size_t goff = (size_t)g * (uint32_t)N * 2u;
 #pragma unroll
@@ -440,8 +441,8 @@ __global__ __launch_bounds__(64 * NWAVE) void w4_stream(WqbmmArgs p, float* __re
             const size_t o = goff + s_lane + (size_t)v * sizeof(SV);
             sv[pc][v] = *reinterpret_cast<const SV*>(static_cast<const char*>(p.scale) + o);
             if (HAS_OFF) ov[pc][v] = *reinterpret_cast<const SV*>(static_cast<const char*>(p.offset) + o);
-            if (!in) sv[pc][v] = (SV)0u;
-            if (HAS_OFF && !in) ov[pc][v] = (SV)0u;
+            if (RAG && !in) sv[pc][v] = (SV)0u;
+            if (RAG && HAS_OFF && !in) ov[pc][v] = (SV)0u;
         }
     }
     constexpr int SL = PF + 1;
@@ -452,7 +453,7 @@ __global__ __launch_bounds__(64 * NWAVE) void w4_stream(WqbmmArgs p, float* __re
         // ahead, or its use moved up, turns the in-order wait into a drain
         __builtin_amdgcn_sched_barrier(0);
         constexpr uint32_t kOutside = 0x80000000u;  // past any buffer here (each is below 2^31 bytes)
-        const bool in = kb * 32 < k_left;
+        const bool in = !RAG || kb * 32 < k_left;
         const uint32_t wl = in ? w_lane : kOutside;
         xa[kb % SL] = __builtin_bit_cast(
             u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, in ? x_lane : kOutside, in ? kb * 64 : 0, 0));
@@ -1013,6 +1014,35 @@ __global__ __launch_bounds__(kThreads) void w4_xsum(WqbmmArgs p, float* __restri
     xsum[t] = s;
 }
 
+// The same for long groups (one group over all of K, say), a wave per (group, row): 16 bytes per lane and load, the
+// lanes' sums added by DPP rotations.  One thread per group reads its whole row by itself: at one group of 4096 on
+// 250-900 rows that was 90-130 us of the call.
+constexpr int64_t kXsumWaveGroup = 512;
+__global__ __launch_bounds__(kThreads) void w4_xsum_wave(WqbmmArgs p, float* __restrict__ xsum) {
+    const int64_t M = p.M, G = p.group, ng = p.K / G;
+    const int64_t t = (int64_t)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
+    if (t >= M * ng) return;
+    const int64_t g = t / M, m = t - g * M;
+    const int lane = threadIdx.x & 63;
+    const uint16_t* row = static_cast<const uint16_t*>(p.x) + m * p.K + g * G;
+    float s = 0.0f;
+    for (int64_t k0 = 8 * lane; k0 < G; k0 += 4 * 512) {  // G is a multiple of 64: whole 8-element pieces
+        u32x4 v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            v[j] = k0 + 512 * j < G ? *reinterpret_cast<const u32x4*>(row + k0 + 512 * j) : (u32x4){0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                s += load_half_bits(v[j][e] & 0xffffu, p.x_dtype);
+                s += load_half_bits(v[j][e] >> 16, p.x_dtype);
+            }
+    }
+    s = wave_sum(s);
+    if (lane == 0) xsum[t] = s;
+}
+
 // Prefill on whole tiles (M % 256 == 0, N % 128 == 0, G % 64 == 0): the tile
 // and MFMA layout of w4_gemm and its group algebra, with a deeper pipeline
 // and the group sums of x taken from w4_xsum instead of a ones-vector MFMA
@@ -1465,10 +1495,11 @@ hipError_t launch_decode_dt(const WqbmmArgs& p, const DecodePlan& d, float* part
 struct StreamPlan {
     bool ok;
     int wpl, nwave, nkb, pf, nsplit, nstrip, piece_kb;
+    bool ragged;  // the last split reaches past K
 };
 
 StreamPlan stream_plan(const WqbmmArgs& p) {
-    StreamPlan s{false, 16, 8, 4, 2, 1, 0, 4};
+    StreamPlan s{false, 16, 8, 4, 2, 1, 0, 4, false};
     const int64_t G = p.group == 0 ? p.K : p.group;
     const bool w8 = p.w_dtype == QK_I8;
     if (!(p.w_dtype == QK_I32 || (w8 && p.N % 4 == 0)) || p.M <= 0 || p.M > 16 || p.N <= 0 || p.K <= 0) return s;
@@ -1535,6 +1566,7 @@ StreamPlan stream_plan(const WqbmmArgs& p) {
     if (p.K % (kw * rows) != 0 || (kw * halves != 8 && kw * halves != 16) || (w8 && kw != kw_full)) kw = kw_full;
     s.nwave = kw * halves;
     s.nsplit = (int)((p.K + kw * rows - 1) / (kw * rows));
+    s.ragged = p.K % (kw * rows) != 0;
     s.nstrip = (int)((p.N + 255) / 256);
     if (s.nsplit > 1 && (int64_t)s.nsplit * p.M * p.N * 4 > ((int64_t)256 << 20)) return s;
     s.ok = (int64_t)s.nstrip * s.nsplit < ((int64_t)1 << 31);
@@ -1545,12 +1577,12 @@ template <int DT, int NWAVE, int NKB, int PF, int PKB, bool HAS_OFF, bool W8, in
 hipError_t launch_stream_t(const WqbmmArgs& p, const StreamPlan& s, float* partial, uint64_t* ctr,
                            hipStream_t stream) {
     const dim3 grid((uint32_t)((int64_t)s.nstrip * s.nsplit));
-    if (s.nsplit == 1)
-        w4_stream<DT, WPL, NWAVE, NKB, PF, PKB, HAS_OFF, true, W8><<<grid, dim3(64 * NWAVE), 0, stream>>>(
-            p, partial, s.nstrip, 1, nullptr, 0);
-    else
-        w4_stream<DT, WPL, NWAVE, NKB, PF, PKB, HAS_OFF, false, W8><<<grid, dim3(64 * NWAVE), 0, stream>>>(
-            p, partial, s.nstrip, s.nsplit, ctr, ctr ? next_split_tag() : 0);
+    const auto k = s.ragged ? (s.nsplit == 1 ? w4_stream<DT, WPL, NWAVE, NKB, PF, PKB, HAS_OFF, true, W8, true>
+                                             : w4_stream<DT, WPL, NWAVE, NKB, PF, PKB, HAS_OFF, false, W8, true>)
+                            : (s.nsplit == 1 ? w4_stream<DT, WPL, NWAVE, NKB, PF, PKB, HAS_OFF, true, W8>
+                                             : w4_stream<DT, WPL, NWAVE, NKB, PF, PKB, HAS_OFF, false, W8>);
+    if (s.nsplit == 1) ctr = nullptr;
+    k<<<grid, dim3(64 * NWAVE), 0, stream>>>(p, partial, s.nstrip, s.nsplit, ctr, ctr ? next_split_tag() : 0);
     return hipGetLastError();
 }
 
@@ -1638,8 +1670,8 @@ template <int DT, bool OFF>
 hipError_t launch_gemm_t(const WqbmmArgs& p, const GemmPlan& g, float* xsum, hipStream_t stream) {
     const dim3 grid((uint32_t)(g.tiles_m * g.tiles_n));
     if (g.dma) {
-        const int64_t sums = p.M * (p.K / p.group);
-        w4_xsum<<<dim3((uint32_t)((sums + kThreads - 1) / kThreads)), dim3(kThreads), 0, stream>>>(p, xsum);
+        const hipError_t e = launch_w4_xsum(p, xsum, stream);
+        if (e != hipSuccess) return e;
         if (p.w_dtype == QK_I8) w4_dma<DT, OFF, true><<<grid, dim3(pd::NT), 0, stream>>>(p, g.tiles_m, g.tiles_n, xsum);
         else w4_dma<DT, OFF, false><<<grid, dim3(pd::NT), 0, stream>>>(p, g.tiles_m, g.tiles_n, xsum);
     } else if (p.w_dtype == QK_I8) {
@@ -1677,6 +1709,11 @@ hipError_t launch_reduce(const WqbmmArgs& p, int nsplit, const float* partial, h
 
 hipError_t launch_w4_xsum(const WqbmmArgs& p, float* xsum, hipStream_t stream) {
     const int64_t sums = p.M * (p.K / p.group);
+    if (p.group >= kXsumWaveGroup) {
+        constexpr int64_t per = kThreads / 64;
+        w4_xsum_wave<<<dim3((uint32_t)((sums + per - 1) / per)), dim3(kThreads), 0, stream>>>(p, xsum);
+        return hipGetLastError();
+    }
     w4_xsum<<<dim3((uint32_t)((sums + kThreads - 1) / kThreads)), dim3(kThreads), 0, stream>>>(p, xsum);
     return hipGetLastError();
 }
