@@ -399,6 +399,7 @@ __device__ __forceinline__ void qmm_store(const QmmEpilogue& e, int64_t m, int64
 //   w4nz_nit=<1..32>                                NZ decode kernel: 128-row superblocks per wave (up to 8, K/128
 //                                                   splitting evenly into at most 16 waves of them; else the
 //                                                   ragged form)
+//   nz_mid=<0|1..16|on>                             NZ mid-M kernel: 0 never; n K splits; on: every shape it takes
 //   w4nz_ragged=1                                   NZ decode kernel: the ragged form for every shape
 struct PlanOverride {
     int w4_stream_nwave = 0, w4_stream_nkb = 0, w4_stream_pf = 0;  // 0: the planner's choice
@@ -419,6 +420,7 @@ struct PlanOverride {
     int qmm_small = -1;
     int w4nz_wg = 0, w4nz_nit = 0;
     bool w4nz_ragged = false;
+    int nz_mid = -1;  // -1 the planner's choice, 0 never, 1..16 that split, 17 every shape
 };
 const PlanOverride& plan_override();
 // CUs of the current device (cached per device; 0 if it cannot be read)
@@ -491,6 +493,10 @@ size_t w4_nz_workspace(const WqbmmArgs& args, bool stream_k = true);
 size_t w4_cast_nz_workspace(const WqbmmArgs& args, bool stream_k = true);
 bool launch_w4_cast_nz(const WqbmmArgs& args, void* workspace, size_t ws_bytes, hipStream_t stream, hipError_t* err);
 hipError_t launch_w4_nz_bmm(const WqbmmArgs& args, void* workspace, size_t ws_bytes, hipStream_t stream);
+// The mid-M kernel on NZ (int4, int8) and int8 [N, K] weights (nz_mid.hip; args.group resolved, not 0).
+double nz_mid_estimate(const WqbmmArgs& args);  // us; negative where it does not take the call
+size_t nz_mid_workspace(const WqbmmArgs& args);
+hipError_t launch_nz_mid(const WqbmmArgs& args, void* workspace, size_t ws_bytes, hipStream_t stream);
 
 // Static quantization (static_quant.hip): x [outer][C][inner] (fp32/fp16/bf16) -> q (int8/uint8/int32);
 // scales == nullptr: per tensor with scale0 / zp0.

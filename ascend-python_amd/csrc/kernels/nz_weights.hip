@@ -1226,7 +1226,54 @@ bool nz_chunks_ok(const WqbmmArgs& p) {
     return nz_plan(c).ok;
 }
 
+// The mid-M kernel (nz_mid.hip) is taken where its estimate is below the kernel's that would run otherwise, in us:
+//   decode kernel: every CU runs one workgroup at a time, and each of the 16-row blocks reads the weight again, so
+//     rounds of workgroups x superblocks per wave x (1.35 + c per block), c = 0.35 int4, 0.8 int8 NZ, 1.3 [N, K]
+//     (N = 11008, K = 4096, M = 20 / 40 12.2 / 17.4 measured; K = 11008, N = 4096, M = 64 40.8; K = 28672, N = 8192,
+//     M = 60 102; [N, K], N = 11008, K = 4096, M = 23 23.4);
+//   prefill kernel: 2.05 per 128-row int4 step (1.15 per 64-row int8 step) of one round of 128 x 256 tiles, and about
+//     8 of its launches (N = 11008, K = 4096, M = 250 / 400 66.8 / 67.9 against 45.8 / 52.4; N = 28672, M = 250 69.0
+//     against 90.7); from a tile per CU on it is ahead (N = 11008, M = 900 / 2000 102.7 / 197.9 against 111.5 / 226.1).
+//     An [N, K] weight is transposed and cast before it, which weighs in at any M (M = 900 316 against 139).
+// Shapes neither takes are unpacked for the row-major kernels and always run the mid-M kernel where it can.
+double nz_decode_estimate(const WqbmmArgs& p) {
+    const NzPlan z = nz_plan(p);
+    if (!z.ok) return -1.0;
+    const double c = p.w_dtype == QK_I4_NZ ? 0.35 : p.w_dtype == QK_I8_NZ ? 0.8 : 1.3;
+    return (double)(((int64_t)z.nwg * z.nrb + 255) / 256) * z.nit * (1.35 + c * z.nb) + 2.0;
+}
+
+bool nz_mid_wanted(const WqbmmArgs& p) {
+    const int ov = plan_override().nz_mid;  // debug override: never, or wherever it can
+    if (ov == 0 || p.M <= 16) return false;
+    const double t = nz_mid_estimate(p);
+    if (t < 0) return false;
+    if (ov > 0) return true;
+    if (p.M <= kNzChunkRows) {
+        const double d = nz_decode_estimate(p);
+        return d < 0 || t < d;
+    }
+    if (nz_chunks_ok(p)) {
+        WqbmmArgs c = p;
+        c.M = kNzChunkRows;
+        double d = nz_decode_estimate(c) * (double)(p.M / kNzChunkRows);
+        if ((c.M = p.M % kNzChunkRows) > 0) d += nz_decode_estimate(c);
+        return t < d;
+    }
+    WqbmmArgs q = p;
+    if (p.w_dtype == QK_I8_NK) q.w_dtype = QK_I8_NZ;
+    const NzGemmPlan g = nzg_plan(q);
+    if (!g.ok) return true;
+    const bool w8 = p.w_dtype != QK_I4_NZ;
+    const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n;
+    if (tiles >= 256 && p.w_dtype != QK_I8_NK) return false;
+    const double steps = (double)p.K / (w8 ? nzg::KS8 : nzg::KS), rounds = tiles < 256 ? 1.0 : (double)tiles / 256.0;
+    const double casts = p.w_dtype == QK_I8_NK ? 4.0 + 0.9e-6 * (double)(p.K * p.N) : 0.0;
+    return t < rounds * steps * (w8 ? 1.15 : 2.05) + 8.0 + casts;
+}
+
 size_t w4_nz_workspace(const WqbmmArgs& p, bool stream_k) {
+    if (stream_k && nz_mid_wanted(p)) return nz_mid_workspace(p);  // a launch given less runs the kernels below
     // the decode kernel needs none; with 64-row groups the query keeps reporting the room of the ND form
     const NzPlan z = plan_override().w4nz_off ? NzPlan{} : nz_plan(p);
     if (z.ok && z.sub == 1) return 0;
@@ -1238,6 +1285,8 @@ size_t w4_nz_workspace(const WqbmmArgs& p, bool stream_k) {
 }
 
 hipError_t launch_w4_nz_bmm(const WqbmmArgs& p, void* workspace, size_t ws_bytes, hipStream_t stream) {
+    if (nz_mid_wanted(p) && (nz_mid_workspace(p) == 0 || (workspace && ws_bytes >= nz_mid_workspace(p))))
+        return launch_nz_mid(p, workspace, ws_bytes, stream);
     const NzPlan z = plan_override().w4nz_off ? NzPlan{} : nz_plan(p);
     if (z.ok)
         return p.x_dtype == QK_BF16 ? launch_nz_dt<QK_BF16>(p, z, stream) : launch_nz_dt<QK_F16>(p, z, stream);
@@ -1311,12 +1360,36 @@ bool cast_nz_decode(const WqbmmArgs& p) {
     return nz_decode_ok(q);
 }
 
+// Row-major weights that the mid-M kernel, or up to 64 rows of int4 the NZ decode kernel where it is ahead of that,
+// runs on after the cast: q, the call on the cast weight.  int8 from 33 rows, as for
+// the other kernels below.  int4 up to 256 rows has row-major kernels, so the cast (6.5 us and 0.22 per MB of weight)
+// and the kernel are weighed against them: the 16-row-block decode kernel at 8 us and 0.22 per MB and row block (N =
+// 4096, K = 4096, M = 20 / 100 / 250 10.6 / 22.5 / 36.3 us against 19.2 / 25.1 / 29.5; N = 13696, K = 5120 29.2 / 62.5
+// / 127.7 against 34.2 / 52.4 / 76.0), the register-staged prefill kernel at 1.75 us per 64-row step and round of its
+// 256 x 128 tiles (N = 32000, K = 4096, M = 20-100 114-119 us against 53-80; it also takes every K of no whole 256
+// rows: K = 11008 92 us against 26-49).
+bool cast_nz_mid(const WqbmmArgs& q) {
+    if (q.w_dtype == QK_I8_NZ) return q.M > 32 && nz_mid_wanted(q);
+    if (plan_override().nz_mid == 0) return false;
+    const bool mid = nz_mid_wanted(q);
+    if (mid && (q.M > 256 || plan_override().nz_mid > 0)) return true;
+    if (q.M <= 16 || (!mid && !(q.M <= kNzChunkRows && nz_plan(q).ok))) return false;
+    const double mb = 0.5e-6 * (double)(q.K * q.N);
+    const int64_t tiles = (q.M + 255) / 256 * ((q.N + 127) / 128);
+    const bool blocks = q.K % 256 == 0 && tiles < 128;
+    const double rows = blocks ? 8.0 + 0.22 * mb * (double)((q.M + 15) / 16)
+                               : 1.75 * (double)(q.K / 64) * (double)((tiles + 255) / 256);
+    return (mid ? nz_mid_estimate(q) : nz_decode_estimate(q)) + 6.5 + 0.22 * mb < rows;
+}
+
 size_t w4_cast_nz_workspace(const WqbmmArgs& p, bool stream_k) {
     const PlanOverride& ov = plan_override();
     if (!(p.w_dtype == QK_I32 || p.w_dtype == QK_I8) || ov.w4nz_off || ov.w4_gemm != 0) return 0;
     WqbmmArgs q = p;
     q.w = reinterpret_cast<const void*>((uintptr_t)256);  // the cast's destination: 256-byte aligned
     q.w_dtype = p.w_dtype == QK_I8 ? QK_I8_NZ : QK_I4_NZ;
+    if (stream_k && cast_nz_mid(q))  // [counters][NZ weight][the mid-M kernel's workspace]
+        return round256(QK_SPLIT_COUNTER_BYTES + round256(nd_weight_bytes(q)) + (nz_mid_wanted(q) ? nz_mid_workspace(q) : 0));
     if (cast_nz_decode(p)) return round256(QK_SPLIT_COUNTER_BYTES + round256(nd_weight_bytes(q)));
     if (p.M < cast_nz_min_m(p.w_dtype) || !nzg_plan(q).ok) return 0;
     return round256(QK_SPLIT_COUNTER_BYTES + round256(nd_weight_bytes(q)) +
@@ -1324,14 +1397,23 @@ size_t w4_cast_nz_workspace(const WqbmmArgs& p, bool stream_k) {
 }
 
 bool launch_w4_cast_nz(const WqbmmArgs& p, void* workspace, size_t ws_bytes, hipStream_t stream, hipError_t* err) {
-    const size_t need = w4_cast_nz_workspace(p, false);
-    if (need == 0 || !workspace || ws_bytes < need || (uintptr_t)workspace % 256 != 0) return false;
+    const size_t full = w4_cast_nz_workspace(p, true), need = w4_cast_nz_workspace(p, false);
+    if (full == 0 || !workspace || (uintptr_t)workspace % 256 != 0) return false;
     char* ws = static_cast<char*>(workspace);
     void* nz = ws + QK_SPLIT_COUNTER_BYTES;
     const bool w8 = p.w_dtype == QK_I8;
     WqbmmArgs q = p;
     q.w = nz;
     q.w_dtype = w8 ? QK_I8_NZ : QK_I4_NZ;
+    if (ws_bytes >= full && cast_nz_mid(q)) {
+        hipError_t e = w8 ? launch_w8_nz_cast(static_cast<const int8_t*>(p.w), true, p.K, p.N, static_cast<int8_t*>(nz), stream)
+                          : launch_w4_nz_cast(static_cast<const int32_t*>(p.w), true, p.K, p.N, static_cast<int32_t*>(nz), stream);
+        const size_t used = QK_SPLIT_COUNTER_BYTES + round256(nd_weight_bytes(q));
+        if (e == hipSuccess) e = launch_w4_nz_bmm(q, ws + used, ws_bytes - used, stream);
+        *err = e;
+        return true;
+    }
+    if (need == 0 || ws_bytes < need) return false;
     if (cast_nz_decode(p)) {
         if (!nz_decode_ok(q)) return false;  // with the call's own operands (their alignment)
         hipError_t e = launch_w8_nz_cast(static_cast<const int8_t*>(p.w), true, p.K, p.N, static_cast<int8_t*>(nz),

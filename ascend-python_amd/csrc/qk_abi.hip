@@ -100,6 +100,10 @@ bool parse_plan(const char* spec, PlanOverride& o) {
             r.w4nz_wg = a;
         } else if (k == "w4nz_nit" && std::sscanf(v.c_str(), "%d", &a) == 1 && a >= 1 && a <= 32) {
             r.w4nz_nit = a;
+        } else if (k == "nz_mid" && v == "on") {
+            r.nz_mid = 17;
+        } else if (k == "nz_mid" && std::sscanf(v.c_str(), "%d", &a) == 1 && a >= 0 && a <= 16) {
+            r.nz_mid = a;
         } else if (k == "w4nz_ragged" && v == "1") {
             r.w4nz_ragged = true;
         } else if (k == "skinny_pf" && (v == "1" || v == "2" || v == "3")) {
