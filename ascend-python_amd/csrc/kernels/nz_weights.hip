@@ -968,12 +968,14 @@ NzPlan nz_plan(const WqbmmArgs& p) {
     // M = 1: 12.1 / 9.7; K = 8192, N = 8192 int8: 17.8 / 15.1), and where the even form's registers hold fewer
     // blocks than a workgroup per CU needs (M = 16: K = 5120, N = 13696 17.9 / 12.7; K = 8192, N = 28672 36.1 /
     // 32.7, int8 64.9 / 55.7).  Elsewhere the unrolled even form is ahead (M = 16: K = 8192, N = 3584 9.0 / 10.2,
-    // K = 5120, N = 1536 6.7 / 7.8), also for [N, K] rows (K = 5120, N = 13696, M = 9: 31.5 / 36.7) and for one
-    // row block of an int8 weight on fewer than 16 waves (the same shape, M = 8: 23.6 / 25.0).
+    // K = 5120, N = 1536 6.7 / 7.8), also for [N, K] rows (K = 5120, N = 13696, M = 9: 31.5 / 36.7; on fewer
+    // than 16 waves also up to 4 rows, N = 13696, M = 3: 28.9 / 31.8, N = 1536, M = 1: 6.8 / 7.3) and for one row
+    // block of an int8 weight on fewer than 16 waves (the same shape, M = 8: 23.6 / 25.0).
     if (nit > 2 && ov.w4nz_nit == 0) {
         const bool held = nb <= nz_max_blocks(nit, w8) || p.w_dtype == QK_I8_NK ||
                           (w8 && z.nrb == 1 && S / nit < kNzMaxWaves);
-        if (p.M <= 4 || !held) nit = 0;
+        const bool few_nk = p.w_dtype == QK_I8_NK && S / nit < kNzMaxWaves;
+        if ((p.M <= 4 && !few_nk) || !held) nit = 0;
     }
     if (nit == 0) {
         z.ragged = true;
