@@ -23,8 +23,10 @@
 //
 // Decode kernel (w4nz_decode), M <= 64: each workgroup owns a few n-blocks
 // over all of K, so no partial sums leave the workgroup.  Its waves split K
-// into equal runs of superblocks; every wave issues the loads of two
-// superblocks ahead (for K = 4096 that is all of its loads, issued before the
+// into equal runs of superblocks (even form) or runs of one length with a
+// shorter last one (ragged form: any K, 64-row groups); every wave issues the
+// loads of two (ragged, up to 4 rows: four) superblocks ahead (for K = 4096
+// that is all of its loads, issued before the
 // first MFMA; x by whole-line DMAs into the wave's LDS slots, the weights
 // non-temporal), folds group scale and offset into its accumulators per
 // superblock with the algebra of the row-major kernels,
@@ -1054,8 +1056,8 @@ size_t nd_weight_bytes(const WqbmmArgs& p) {
     return (size_t)(p.w_dtype == QK_I8_NZ || p.w_dtype == QK_I8_NK ? p.K * p.N : p.K * p.N / 2);
 }
 
-// Prefill plan on an int4 NZ weight: M > 64 with at least 96 tiles of 128 x 256, N % 256 == 0, groups of
-// whole 128-row NZ blocks, 16-byte aligned operands and 32-bit buffer offsets.  The workspace holds the x
+// Prefill plan on an NZ weight: M > 64 with at least 64 tiles of 128 x 256, N % 256 == 0, groups of whole
+// K steps (128 rows of an int4 weight, 64 of an int8 one), 16-byte aligned operands and 32-bit buffer offsets.  The workspace holds the x
 // group sums ([split counters, unused][fp32 [K/G][M]]).
 struct NzGemmPlan {
     bool ok;
@@ -1198,13 +1200,15 @@ hipError_t launch_w8_nz_cast(const int8_t* src, bool to_nz, int64_t K, int64_t N
     return hipGetLastError();
 }
 
-// NZ weights (int4 QK_I4_NZ, int8 QK_I8_NZ): the decode kernel where it applies (no workspace);
+// NZ weights (int4 QK_I4_NZ, int8 QK_I8_NZ): the decode kernel where it applies (no workspace), the mid-M kernel
+// or the prefill kernel (nz_mid_wanted weighs them);
 // otherwise the weight is unpacked into the workspace and the row-major kernels run on it:
 // [QK_SPLIT_COUNTER_BYTES, unused][ND weight][row-major call's workspace].
 // An int8 [N, K] weight (QK_I8_NK) takes the same decode kernel (reading it in place) or is transposed into the
 // workspace for the row-major kernels: [QK_SPLIT_COUNTER_BYTES, unused][[K, N] weight][row-major call's workspace].
 // int8 NZ / [N,K] weights with 64 < M <= 192, or up to 256 where the NZ prefill kernel does not take the shape
-// (it needs 64 tiles): the decode kernel on row chunks of at most 64, no workspace.  The alternative unpacks the
+// (it needs 64 tiles), where the mid-M kernel does not run (a workspace too small for its splits, or its estimate):
+// the decode kernel on row chunks of at most 64, no workspace.  The alternative unpacks the
 // weight and runs the row-major int8 kernels (N = 4096, K = 4096: M = 65 / 128 68 / 103 us, against ~2 x 21 us;
 // M = 129-256 ~130 us against 3-4 x 21 us).  int4 keeps the unpack, which is faster there (28-35 us against
 // ~2 x 19 us).
@@ -1344,14 +1348,16 @@ hipError_t launch_w4_nz_bmm(const WqbmmArgs& p, void* workspace, size_t ws_bytes
 // kernels: int4 M = 257 / 384 / 512 / 640 / 896 86 / 79 / 80 / 84 / 111 us against 126 / 120 / 87 / 228 / 234 us
 // (the row-major prefill kernel's register-staged form takes a ragged M), while at M = 200 / 256 the decode
 // kernels are faster (67 / 72 against 77 us); int8 M = 200 / 256 / 384 / 640 116 / 117 / 116 / 120 us against
-// 6450 / 7927 / 126 / 246 us.  So int4 casts from M = 257 and int8 from M = 129.  The debug overrides that
+// 6450 / 7927 / 126 / 246 us.  So for the prefill kernel int4 casts from M = 257 and int8 from M = 129 (the mid-M
+// kernel has its own rule, cast_nz_mid).  The debug overrides that
 // force or disable a prefill kernel switch it off.
 int64_t cast_nz_min_m(int w_dtype) { return w_dtype == QK_I8 ? 129 : 257; }
 
 // An int8 row-major weight with 32 < M <= 128 (or up to 256 where the NZ prefill kernel does not take the shape)
 // is cast too, for the NZ decode kernel (on row chunks past 64 rows): N = 4096, K = 4096, M = 65 / 128 41 / 53 us
 // against 68 / 90 us for the row-major decode stream on 16-row slices; at N = 11008 60 / 80 against 68 / 107 us.
-// The call's workspace then holds the NZ weight alone.
+// The call's workspace then holds the NZ weight alone.  Where the mid-M kernel is ahead of the decode kernel it runs
+// on the cast weight instead, if its workspace is there (cast_nz_mid).
 bool nz_decode_ok(const WqbmmArgs& q) { return q.M <= kNzChunkRows ? nz_plan(q).ok : nz_chunks_ok(q); }
 
 bool cast_nz_decode(const WqbmmArgs& p) {

@@ -29,11 +29,12 @@
  * contents -- uninitialised memory is fine.  A non-empty workspace begins with
  * QK_SPLIT_COUNTER_BYTES of split-K arrival counters, followed by the partial
  * sums (split-K shapes) or by the activations' per-group sums (weight-quant
- * matmul at large M; from M = 257 on a row-major int4 weight, and from M = 33
- * on a row-major int8 weight, the weight cast to NZ, K*N/2 (int4) or K*N
- * (int8) bytes rounded to 256, comes first, then the sums (none up to M = 128
- * on int8, where the NZ decode kernel runs); where the NZ
- * prefill kernel runs stream-K, (P - 1) x 128 KB of fp32 partial slots follow
+ * matmul at large M; where a row-major weight is cast per call -- from M = 17
+ * on an int4 weight where that is faster, from M = 33 on an int8 weight -- the
+ * weight cast to NZ, K*N/2 (int4) or K*N
+ * (int8) bytes rounded to 256, comes first, then the sums or the fp32 partial
+ * tiles of the mid-M kernel's K splits (none where the NZ decode kernel runs);
+ * where the NZ prefill kernel runs stream-K, (P - 1) x 128 KB of fp32 partial slots follow
  * the sums, P being the current device's CU count).  Each arrival adds D = tag * 2^16 + 1 to its
  * counter (a 48-bit tag drawn per call, never 0 or all ones), so a counter of
  * this call holds j * D after j arrivals; a zero word is empty (the last
@@ -237,8 +238,9 @@ int qk_weight_quant_bmm(const void* x, int x_dtype,
  * reports fits in that array, the call runs exactly the kernels qk_weight_quant_bmm
  * runs (the same bits).  Where only the NZ prefill kernel's stream-K partial
  * slots do not fit, it runs that kernel with whole tiles per workgroup (the
- * same bits again).  Otherwise, for a row-major int4 weight at M >= 257 or int8
- * weight at M >= 33 whose cast to NZ is what does not fit, it runs the
+ * same bits again); where the mid-M kernel's K splits do not fit, the kernels
+ * without it (within 1e-2).  Otherwise, for a row-major int4 weight at M >= 17
+ * or int8 weight at M >= 33 whose cast to NZ is what does not fit, it runs the
  * row-major kernels without the cast (within the same 1e-2 bar; for int4 on
  * cfg3's shape, N = 11008, K = 4096, 128-row groups, at M = 1024 and 2048 the
  * same bits); a shape whose scratch exceeds
