@@ -942,6 +942,8 @@ __global__ __launch_bounds__(dm::NT) void qmm_dma(QmmArgs p, int tiles_m, int ti
 // stages' global loads in flight in registers.  With several splits each writes exact int32
 // partial sums and qmm_reduce adds them (order-free, exact) before the same
 // epilogue as every other path.
+// HALF: [K,N] rows of 8-byte alignment (N = 1000): each 16-byte piece of a weight row is read as two halves, the
+// second one only inside N.  A form of its own, so that aligned rows keep their single load.
 namespace sk {
 constexpr int BN = 256, BK = 128;
 __host__ __device__ __forceinline__ int64_t sk_k_len(int64_t K, int64_t nsplit) {
@@ -949,7 +951,7 @@ __host__ __device__ __forceinline__ int64_t sk_k_len(int64_t K, int64_t nsplit) 
 }
 }
 
-template <bool B_KN, int MT, bool FINAL, int PF = 1>
+template <bool B_KN, int MT, bool FINAL, int PF = 1, bool HALF = false>
 __global__ __launch_bounds__(kThreads) void qmm_skinny(QmmArgs p, int tiles_n, int nsplit, int32_t* partial) {
     using big::rk_off;
     using big::kn_off;
@@ -1000,7 +1002,18 @@ __global__ __launch_bounds__(kThreads) void qmm_skinny(QmmArgs p, int tiles_n, i
             } else {
                 const int kr = q >> 4, c16 = q & 15;
                 const int64_t n = n0 + 16 * c16;
-                rb[sl][i] = n < p.N ? wload(p.b + (k0 + kr) * p.sbk + n) : (i32x4){0, 0, 0, 0};
+                if constexpr (HALF) {
+                    auto hload = [&](int64_t nh) {
+                        const i32x2* v = reinterpret_cast<const i32x2*>(p.b + (k0 + kr) * p.sbk + nh);
+                        if (nh >= p.N) return (i32x2){0, 0};
+                        if constexpr (MT == 1) return __builtin_nontemporal_load(v);
+                        else return *v;
+                    };
+                    const i32x2 lo = hload(n), hi = hload(n + 8);
+                    rb[sl][i] = (i32x4){lo[0], lo[1], hi[0], hi[1]};
+                } else {
+                    rb[sl][i] = n < p.N ? wload(p.b + (k0 + kr) * p.sbk + n) : (i32x4){0, 0, 0, 0};
+                }
             }
         }
     };
@@ -1882,20 +1895,24 @@ SkinnyPlan skinny_plan(int64_t M, int64_t N, int64_t K) {
     return s;
 }
 
-template <bool B_KN, int MT>
+template <bool B_KN, int MT, bool HALF>
 hipError_t launch_skinny_t(const QmmArgs& p, const SkinnyPlan& s, int32_t* partial, hipStream_t stream) {
     const dim3 grid((uint32_t)((int64_t)s.tiles_m * s.tiles_n * s.nsplit));
     if (s.nsplit == 1) {
         // 128-row tiles run only as a split stream (skinny_plan), so that instance is not built
         if constexpr (MT == 8) return hipErrorInvalidValue;
-        else {
+        else if constexpr (HALF) {  // at the plan's own depth
+            qmm_skinny<B_KN, MT, true, MT == 1 ? 2 : 1, true><<<grid, dim3(kThreads), 0, stream>>>(p, s.tiles_n, 1, nullptr);
+            return hipGetLastError();
+        } else {
             const auto k = s.pf == 3 ? qmm_skinny<B_KN, MT, true, 3>
                            : s.pf == 2 ? qmm_skinny<B_KN, MT, true, 2> : qmm_skinny<B_KN, MT, true, 1>;
             k<<<grid, dim3(kThreads), 0, stream>>>(p, s.tiles_n, 1, nullptr);
             return hipGetLastError();
         }
     }
-    const auto k = s.pf == 3 ? qmm_skinny<B_KN, MT, false, 3>
+    const auto k = HALF ? qmm_skinny<B_KN, MT, false, MT == 1 ? 2 : 1, HALF>
+                   : s.pf == 3 ? qmm_skinny<B_KN, MT, false, 3>
                    : s.pf == 2 ? qmm_skinny<B_KN, MT, false, 2> : qmm_skinny<B_KN, MT, false, 1>;
     k<<<grid, dim3(kThreads), 0, stream>>>(p, s.tiles_n, s.nsplit, partial);
     hipError_t e = hipGetLastError();
@@ -1907,13 +1924,13 @@ hipError_t launch_skinny_t(const QmmArgs& p, const SkinnyPlan& s, int32_t* parti
     return hipGetLastError();
 }
 
-template <bool B_KN>
+template <bool B_KN, bool HALF = false>
 hipError_t launch_skinny(const QmmArgs& p, const SkinnyPlan& s, int32_t* partial, hipStream_t stream) {
     switch (s.mt) {
-    case 1: return launch_skinny_t<B_KN, 1>(p, s, partial, stream);
-    case 2: return launch_skinny_t<B_KN, 2>(p, s, partial, stream);
-    case 4: return launch_skinny_t<B_KN, 4>(p, s, partial, stream);
-    default: return launch_skinny_t<B_KN, 8>(p, s, partial, stream);
+    case 1: return launch_skinny_t<B_KN, 1, HALF>(p, s, partial, stream);
+    case 2: return launch_skinny_t<B_KN, 2, HALF>(p, s, partial, stream);
+    case 4: return launch_skinny_t<B_KN, 4, HALF>(p, s, partial, stream);
+    default: return launch_skinny_t<B_KN, 8, HALF>(p, s, partial, stream);
     }
 }
 
@@ -2152,10 +2169,17 @@ hipError_t launch_quant_matmul(const QmmArgs& p, void* workspace, size_t ws_byte
         if (ok) return b_kn16 ? launch_mid<kLayKN>(p, mp, partial, ctr, stream) : launch_mid<kLayNK>(p, mp, partial, ctr, stream);
         if (p.N % 64 == 0 && p.K % md::KS == 0) return launch_qmm_fallback(p, a_ok, b_kn, b_nk, stream);
     }
-    if (sp.mt != 0 && a_ok && (b_nk || b_kn16)) {
+    // [K,N] rows of 8-byte alignment (N = 1000, 13704): the split stream's half-piece form where the tiled kernel's
+    // serial K loop costs more than the split's second launch (us with the quantization, tiled / stream: K = 4096,
+    // N = 1000, M = 1 / 29 / 100 66 / 15, 71 / 15, 93 / 22; K = 4096, N = 32008, M = 16 / 128 88 / 45, 112 / 73;
+    // K = 512, N = 1000, M = 1 / 16 / 40 13.2 / 15.0, 16.3 / 17.2, 21.5 / 17.3; without a split K = 256, M = 40
+    // 17.8 / 23.7, K = 2048 46 / 40)
+    const bool half = b_kn && !b_kn16 && (sp.nsplit > 1 ? p.K > 512 || p.M > 16 : p.K >= 2048);
+    if (sp.mt != 0 && a_ok && (b_nk || b_kn16 || half)) {
         const size_t need = sp.nsplit > 1 ? QK_SPLIT_COUNTER_BYTES + (size_t)sp.nsplit * p.M * p.N * sizeof(int32_t) : 0;
         if (need && (!workspace || ws_bytes < need)) return hipErrorInvalidValue;
-        return b_kn16 ? launch_skinny<true>(p, sp, partial, stream) : launch_skinny<false>(p, sp, partial, stream);
+        if (half) return launch_skinny<true, true>(p, sp, partial, stream);
+        return b_kn ? launch_skinny<true>(p, sp, partial, stream) : launch_skinny<false>(p, sp, partial, stream);
     }
     BigPlan bp = big_plan(p.M, p.N, p.K);
     bool big_ok = bp.ok && a_ok && (b_nk || (b_kn && p.N % 16 == 0 && p.sbk % 16 == 0 && (uintptr_t)p.b % 16 == 0));

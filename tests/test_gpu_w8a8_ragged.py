@@ -47,6 +47,28 @@ SHAPES = [
 ]
 
 
+# [K,N] rows of 8-byte alignment on the split stream: every row tile, one and two blocks of columns, a last piece of
+# 8 columns, splits of one and several lengths; 8 columns alone; without a split (129 column tiles); and the tiled
+# kernel's side of the rule
+HALF_SHAPES = [
+    (1, 1000, 4096),
+    (16, 264, 1408),
+    (17, 520, 1024),
+    (33, 8, 640),
+    (64, 1000, 13696),
+    (128, 248, 5504),
+    (100, 1000, 4096),
+    (3, 32776, 2048),
+    (16, 1000, 512),
+    (17, 1000, 512),
+]
+
+
+@pytest.mark.parametrize("M,N,K", HALF_SHAPES)
+def test_w8a8_8_byte_rows(ops, oracle, M, N, K):
+    test_w8a8_ragged(ops, oracle, "kn", M, N, K)
+
+
 @pytest.mark.parametrize("layout", ["kn", "nk", "nz"])
 @pytest.mark.parametrize("M,N,K", SHAPES)
 def test_w8a8_ragged(ops, oracle, layout, M, N, K):
@@ -102,3 +124,13 @@ def test_w8a8_nk_columns_of_eight(ops, M, N, K):
     h = ops.npu_quant_matmul(x.to(DEV), w.to(DEV).t(), torch.ones(1, device=DEV), pertoken_scale=pt,
                              output_dtype=torch.bfloat16)
     assert torch.equal(h, (out.float() * pt[:, None]).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("M", [2, 40])
+def test_w8a8_8_byte_column_view(ops, M):
+    """[K,N]: columns 8.. of a wider tensor; rows 16-byte strides apart that start at 8-byte alignment."""
+    g = torch.Generator().manual_seed(M)
+    x = torch.randint(-128, 128, (M, 2048), generator=g, dtype=torch.int8)
+    w = torch.randint(-128, 128, (2048, 288), generator=g, dtype=torch.int8)
+    out = ops.npu_quant_matmul(x.to(DEV), w.to(DEV)[:, 8:280], torch.ones(1, device=DEV), output_dtype=torch.int32)
+    assert np.array_equal(out.cpu().numpy(), (x.double() @ w[:, 8:280].double()).numpy().astype(np.int32))
