@@ -7,8 +7,9 @@
 // all rows by columns 32w .. 32w+31.  The group algebra is the other kernels',
 //   acc += s * sum_k x*(w + BASE) + s*(offset - BASE) * sum_k x,
 // on exact operands.  The group sums of x are taken in the kernel: wave i sums row tile i on the matrix cores (against
-// ones) and hands it to the others through LDS, so a group is folded one step later, row tile by row tile between
-// the next step's first MFMAs.  K is split over workgroups where the tiles alone leave CUs idle: each split stores
+// ones) and hands it to the others through LDS, so a group (128 rows of it, if it is longer) is folded one step later,
+// row tile by row tile between the next step's first MFMAs.  K is split over workgroups where the tiles alone leave
+// CUs idle: each split stores
 // its fp32 sums in the MFMA layout (whole KB per store) and nz_mid_reduce adds them in split order.
 //
 // What bounds it: per step and CU the LDS reads (8 waves x the activation stage: 160 KB at 80 rows), the MFMAs and
@@ -75,7 +76,7 @@ __device__ __forceinline__ void mid_wait(int later) {  // at most `later` steps'
 
 // HALF: an int4 step holds two 64-row groups; each is folded within its step, every wave summing x itself (row tiles
 // of at most 64 rows: more would spill, and a spill's memory operations would break the hand-counted waits).
-// Otherwise a group is one step or several (or all of K).
+// Otherwise a group is one step or several (or all of K), folded every 128 rows.
 
 // wblk / wstep: bytes from one 16-column weight block to the next and from one step to the next; nk: the weight is
 // int8 [N, K] rows (the 16 bytes a lane takes from an NZ block are contiguous in row 16*block + lane%16).
@@ -171,7 +172,7 @@ __global__ __launch_bounds__(nm::NT) void nz_mid(WqbmmArgs p, int tiles_m, int t
 #pragma unroll
     for (int j = 0; j < TN; ++j) sf[j] = sx[j] = 0.0f;
     const int xt = wave % TM;  // the row tile whose sum of x this wave takes: no branch around the MFMAs
-    f32x4 xsum = zero4;        // its running group
+    f32x4 xsum = zero4;        // since the last fold
     for (int e = tid; e < 2 * BM; e += NT) xsbuf[e] = 0.0f;  // what the first fold (of nothing) reads
     const u32x4 ones = {MM::ONES, MM::ONES, MM::ONES, MM::ONES};
     // lane parts of the LDS addresses: a_at[kt] of an activation fragment (row tile i adds i * 16 rows)
@@ -181,7 +182,12 @@ __global__ __launch_bounds__(nm::NT) void nz_mid(WqbmmArgs p, int tiles_m, int t
         a_at[kt] = W8 ? fr * 128 + 16 * ((2 * g4 + kt) ^ (fr & 7)) : fr * 256 + 16 * ((4 * kt + g4) ^ fr);
     constexpr int ROWT = W8 ? 2048 : 4096;  // LDS bytes of 16 rows
 
-    int cleft = 0, cslot = 0;  // steps left of the group being multiplied (0: a group starts)
+    // Raw sums are folded at a group's end, and inside a longer group every 128 rows: at BASE times the size of the
+    // products they would lose what the base's share takes off again (one fp16 group of 5120 rows, positive x, M = 200,
+    // N = 13696: 9.8e-4 off the 64-bit result, folded 2.1e-4, which is the output's rounding).
+    constexpr int FSTEPS = 128 / KSW;
+    int gleft = gsteps - s0 % gsteps, fleft = 0;  // steps left of the group being multiplied, and to its next fold
+    int cslot = 0;
     for (int s = s0; s < s0 + NSTG - 1 && s < s1; ++s) issue(s);
     for (int s = s0; s < s1; ++s) {
         // stage s has landed once at most the later steps' loads are outstanding
@@ -195,9 +201,12 @@ __global__ __launch_bounds__(nm::NT) void nz_mid(WqbmmArgs p, int tiles_m, int t
         const char* Bs = As + XB;
         const char* sc = As + XB + W_BYTES;
         cslot = cslot + 1 < NSTG ? cslot + 1 : 0;
-        const bool first = HALF || cleft == 0;  // a group starts with this step
-        if (!HALF && first) cleft = s == s0 ? gsteps - s0 % gsteps : gsteps;
-        --cleft;
+        const bool first = FSTEPS == 1 || fleft == 0;  // new sums start with this step
+        if (FSTEPS > 1) {
+            if (first) fleft = gleft < FSTEPS ? gleft : FSTEPS;
+            --fleft;
+            if (--gleft == 0) gleft = gsteps;
+        }
         // LDS reads go out ahead of their use: the weight, the factors' raw values, the row tile whose x this wave sums,
         // then each row tile's fragments one tile before its MFMAs.  Row tiles run one after the other over the whole
         // step, so a tile's fold of the previous group (VALU) runs under the MFMAs of the tile before it.
@@ -270,7 +279,7 @@ __global__ __launch_bounds__(nm::NT) void nz_mid(WqbmmArgs p, int tiles_m, int t
                 fold(i, a[1], x[1], f[1], fx[1]);
             }
         } else {
-            auto tiles = [&](auto fresh) {  // fresh: a group starts, so the one before it is folded
+            auto tiles = [&](auto fresh) {  // fresh: new sums start, so those before them are folded
                 constexpr bool F = decltype(fresh)::value;
 #pragma unroll
                 for (int i = 0; i < TM; ++i) {
@@ -292,7 +301,7 @@ __global__ __launch_bounds__(nm::NT) void nz_mid(WqbmmArgs p, int tiles_m, int t
                 tiles(std::true_type());
                 factors(0, sf, sx);
                 xsum = zero4;
-            } else {
+            } else if constexpr (FSTEPS > 1) {
                 tiles(std::false_type());
             }
             // this step's sum of x of row tile xt, for the next step's fold (waves past TM write the same again)

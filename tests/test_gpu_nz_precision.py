@@ -1,0 +1,58 @@
+"""fp32-level error of the weight-quant kernels on NZ and [N, K] weights, on the GPU.
+
+Rows of x come in equal pairs and rows of w in pairs of opposite sign, so every exact output is 0 and the output is
+the error of the kernel's 32-bit sums alone (no 16-bit rounding hides it).  The kernels may sum x * (w + base) raw
+over at most 128 rows before the scale and the base's share, base * sum x, come off: one rounding of such a sum errs
+by at most u = 2^-24 * (base + max|w|) * sum of |x| over 128 rows.  A fold has 8 of them (four MFMAs for the products,
+four for the sum of x) and the K / 128 folds' errors add up as a random walk, so the rms error stays below
+8 * sqrt(K / 128) * u with a margin of about five; raw sums over all of K grow K / 128 times as large and miss it.
+"""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import op_plugin_amd
+    yield op_plugin_amd
+    op_plugin_amd.debug_set_plan("")
+
+
+def _rms_and_bar(ops, int4, layout, M, N, K, group, dtype, base, top, plan):
+    print(f"[case] int4={int4} {layout} M={M} N={N} K={K} G={group} {dtype} plan={plan!r}", flush=True)
+    g = torch.Generator().manual_seed(M + K)
+    x = (0.5 + torch.rand((M, K // 2), generator=g)).to(dtype).repeat_interleave(2, 1)
+    w = torch.randint(-top, top + 1, (K // 2, N), generator=g, dtype=torch.int8).repeat_interleave(2, 0)
+    w[1::2] *= -1
+    if layout == "nk":
+        wd = w.t().contiguous().to(DEV).t()
+    else:
+        wd = ops.npu_convert_weight_to_int4pack(w.to(DEV)) if int4 else w.to(DEV)
+        wd = ops.npu_format_cast(wd, ops.ACL_FORMAT_FRACTAL_NZ) if layout == "nz" else wd
+    s = torch.ones((K // group, N) if group else (N,), dtype=torch.float16, device=DEV)
+    ops.debug_set_plan(plan)
+    out = ops.npu_weight_quant_batchmatmul(x.to(DEV), wd, s, antiquant_group_size=group)
+    ops.debug_set_plan("")
+    u = 2.0 ** -24 * (base + top) * 128 * x.float().mean().item()
+    return out.float().square().mean().sqrt().item(), 8 * math.sqrt(K / 128) * u
+
+
+@pytest.mark.parametrize("layout,M,K,group,dtype,base,plan", [
+    ("nz", 20, 8192, 0, torch.float16, 1032, "nz_mid=1"),
+    ("nz", 64, 8192, 0, torch.float16, 1032, "nz_mid=2"),
+    ("nz", 100, 8192, 1024, torch.float16, 1032, "nz_mid=1"),
+    ("nz", 40, 8192, 0, torch.bfloat16, 136, "nz_mid=1"),
+    ("kn", 70, 8192, 2048, torch.float16, 1032, "nz_mid=1"),
+    ("nz", 16, 8192, 0, torch.float16, 1032, ""),       # the decode kernel
+    ("nz", 3, 128 * 43, 0, torch.float16, 1032, ""),    # its ragged form
+])
+def test_int4_long_groups(ops, layout, M, K, group, dtype, base, plan):
+    rms, bar = _rms_and_bar(ops, True, layout, M, 272, K, group, dtype, base, 7, plan)
+    assert rms <= bar, (rms, bar)
