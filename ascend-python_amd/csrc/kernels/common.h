@@ -48,6 +48,23 @@ struct Mfma<QK_F16> {
     }
 };
 
+// Eight int8 weights (two dwords, eight consecutive rows of one column) as a 16-bit MFMA operand: every int8 is a bf16
+// and an fp16 number, so each byte converts by one sign-extending v_cvt_f32_i32 and is cut (bf16) or packed (fp16)
+// exactly.
+template <int DT>
+__device__ __forceinline__ u32x4 i8_operand(uint32_t lo, uint32_t hi) {
+    const uint32_t w[2] = {lo, hi};
+    u32x4 b;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const uint32_t src = w[q >> 1] >> (16 * (q & 1));
+        const float f0 = (float)(int8_t)src, f1 = (float)(int8_t)(src >> 8);
+        if constexpr (DT == QK_BF16) b[q] = __builtin_amdgcn_perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u);
+        else b[q] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(f0, f1));
+    }
+    return b;
+}
+
 // ---------------------------------------------------------------- conversions
 // fp16 -> fp32 is exact; bf16 -> fp32 is a shift.
 __device__ __forceinline__ float bf16_bits_to_f32(uint32_t b) { return __uint_as_float(b << 16); }

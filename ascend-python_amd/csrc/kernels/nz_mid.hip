@@ -6,11 +6,11 @@
 // rows come into a ring of LDS stages by direct-to-LDS loads, as many steps ahead as the ring holds; wave w multiplies
 // all rows by columns 32w .. 32w+31.  The group algebra is the other kernels',
 //   acc += s * sum_k x*(w + BASE) + s*(offset - BASE) * sum_k x,
-// on exact operands.  The group sums of x are taken in the kernel: wave i sums row tile i on the matrix cores (against
-// ones) and hands it to the others through LDS, so a group (128 rows of it, if it is longer) is folded one step later,
-// row tile by row tile between the next step's first MFMAs.  K is split over workgroups where the tiles alone leave
-// CUs idle: each split stores
-// its fp32 sums in the MFMA layout (whole KB per store) and nz_mid_reduce adds them in split order.
+// on exact operands (BASE = 0 for an int8 weight).  The group sums of x are taken in the kernel: wave i sums row tile i
+// on the matrix cores (against ones) and hands it to the others through LDS, so a group (128 or 512 rows of it, if it is
+// longer) is folded one step later, row tile by row tile between the next step's first MFMAs.  K is split over
+// workgroups where the tiles alone leave CUs idle: each split stores its fp32 sums in the MFMA layout (whole KB per
+// store) and nz_mid_reduce adds them in split order.
 //
 // What bounds it: per step and CU the LDS reads (8 waves x the activation stage: 160 KB at 80 rows), the MFMAs and
 // the fold take about the same time; on few rows the weight stream.
@@ -44,22 +44,6 @@ __device__ __forceinline__ u32x4 mid_op4(uint32_t w) {  // the eight nibbles of 
     return (u32x4){(w & mask) ^ magic, ((w >> 4) & mask) ^ magic, ((w >> 8) & mask) ^ magic, ((w >> 12) & mask) ^ magic};
 }
 
-template <int DT>
-__device__ __forceinline__ u32x4 mid_op8(uint32_t lo, uint32_t hi) {  // eight int8 as exact 16-bit values w + 128
-    const uint32_t flip = __builtin_amdgcn_readfirstlane(0x80808080u);
-    const uint32_t w[2] = {lo ^ flip, hi ^ flip};
-    u32x4 b;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const uint32_t src = w[q >> 1];
-        const float f0 = (float)((src >> (16 * (q & 1))) & 0xffu);
-        const float f1 = (float)((src >> (16 * (q & 1) + 8)) & 0xffu);
-        if constexpr (DT == QK_BF16) b[q] = __builtin_amdgcn_perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u);
-        else b[q] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(f0, f1));
-    }
-    return b;
-}
-
 template <int N, int MOST>
 __device__ __forceinline__ void mid_wait(int later) {  // at most `later` steps' loads (N each, 0 <= later <= MOST <= 4) left
     if (later == MOST) {
@@ -76,7 +60,7 @@ __device__ __forceinline__ void mid_wait(int later) {  // at most `later` steps'
 
 // HALF: an int4 step holds two 64-row groups; each is folded within its step, every wave summing x itself (row tiles
 // of at most 64 rows: more would spill, and a spill's memory operations would break the hand-counted waits).
-// Otherwise a group is one step or several (or all of K), folded every 128 rows.
+// Otherwise a group is one step or several (or all of K).
 
 // wblk / wstep: bytes from one 16-column weight block to the next and from one step to the next; nk: the weight is
 // int8 [N, K] rows (the 16 bytes a lane takes from an NZ block are contiguous in row 16*block + lane%16).
@@ -88,7 +72,7 @@ __global__ __launch_bounds__(nm::NT) void nz_mid(WqbmmArgs p, int tiles_m, int t
     constexpr int KSW = ksw(W8), NKT = KSW / 32, BM = 16 * TM;
     constexpr int XB = x_bytes(TM, W8), STG = stage(TM, W8), NSTG = stages(TM, W8);
     constexpr int XN = XB / 1024, XPW = (XN + 7) / 8;  // activation DMAs per step, and per wave
-    constexpr float BASE = W8 ? 128.0f : MM::BASE;
+    constexpr float BASE = W8 ? 0.0f : MM::BASE;
     static_assert(NSTG >= 3 && NSTG * STG + xs_bytes(TM) <= 160 * 1024 && BM * OROWB <= NSTG * STG, "LDS");
     static_assert(TM <= 6, "one wave sums each row tile; taller tiles would spill, and a spill's memory operations "
                            "would break the hand-counted waits");
@@ -182,10 +166,13 @@ __global__ __launch_bounds__(nm::NT) void nz_mid(WqbmmArgs p, int tiles_m, int t
         a_at[kt] = W8 ? fr * 128 + 16 * ((2 * g4 + kt) ^ (fr & 7)) : fr * 256 + 16 * ((4 * kt + g4) ^ fr);
     constexpr int ROWT = W8 ? 2048 : 4096;  // LDS bytes of 16 rows
 
-    // Raw sums are folded at a group's end, and inside a longer group every 128 rows: at BASE times the size of the
-    // products they would lose what the base's share takes off again (one fp16 group of 5120 rows, positive x, M = 200,
-    // N = 13696: 9.8e-4 off the 64-bit result, folded 2.1e-4, which is the output's rounding).
-    constexpr int FSTEPS = 128 / KSW;
+    // Raw sums are folded at a group's end and inside a longer group: an int4 one every 128 rows, since at BASE times the
+    // size of the products they would lose what the base's share takes off again (one fp16 group of 5120 rows, positive
+    // x, M = 200, N = 13696: 9.8e-4 off the 64-bit result, folded 2.1e-4, which is the output's rounding).  int8 operands
+    // carry no base: every 512 rows keeps the rounding of the long chain low (8192 rows of one group, M = 100, N = 28672:
+    // the 32-bit sums are 1.7e-7 off, at one fold 5.8e-7) for 2-3 % of the time (M = 400, K = 11008, N = 4096: 67.6 us,
+    // one fold 65.2, every 128 rows 72.4).
+    constexpr int FSTEPS = (W8 ? 512 : 128) / KSW;
     int gleft = gsteps - s0 % gsteps, fleft = 0;  // steps left of the group being multiplied, and to its next fold
     int cslot = 0;
     for (int s = s0; s < s0 + NSTG - 1 && s < s1; ++s) issue(s);
@@ -238,7 +225,7 @@ __global__ __launch_bounds__(nm::NT) void nz_mid(WqbmmArgs p, int tiles_m, int t
         for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
-                if constexpr (W8) b[kt][j] = mid_op8<DT>(bw[j][2 * kt], bw[j][2 * kt + 1]);
+                if constexpr (W8) b[kt][j] = i8_operand<DT>(bw[j][2 * kt], bw[j][2 * kt + 1]);
                 else b[kt][j] = mid_op4<MM::MAGIC>(bw[j][kt]);
             }
         auto factors = [&](int u, float (&f)[TN], float (&x)[TN]) {  // s and s * (offset - BASE) of the step's group u

@@ -30,8 +30,8 @@
 // first MFMA; x by whole-line DMAs into the wave's LDS slots, the weights
 // non-temporal), folds group scale and offset into its accumulators per
 // superblock with the algebra of the row-major kernels,
-//   acc += s * sum_k x*(w + BASE) + s*(offset - BASE) * sum_k x,
-// and the waves' sums are added through LDS in K order (deterministic).
+//   acc += s * sum_k x*(w + BASE) + s*(offset - BASE) * sum_k x
+// (int8 operands are the bytes' own values: BASE = 0), and the waves' sums are added through LDS in K order (deterministic).
 #include <atomic>
 
 #include "common.h"
@@ -290,7 +290,7 @@ __device__ __forceinline__ u32x4 nz_operand(uint32_t w) {
     return b;
 }
 
-// Eight int8 weights (two dwords, 8 consecutive rows of one column) as a
+// The prefill kernel's: eight int8 weights (two dwords, 8 consecutive rows of one column) as a
 // 16-bit MFMA operand of offset-binary values u = w + 128 (BASE 128): each
 // byte converts exactly to float (v_cvt_f32_ubyte) and from there to
 // bf16 (the upper half: u <= 255 fits 8 significant bits) or fp16.
@@ -460,7 +460,7 @@ __global__ __launch_bounds__(64 * kNzMaxWaves) void w4nz_decode(WqbmmArgs p, int
     for (int it = 0; it < PF; ++it) issue(it, it);
 
     const u32x4 ones = {MM::ONES, MM::ONES, MM::ONES, MM::ONES};
-    constexpr float BASE = W8 ? 128.0f : MM::BASE;
+    constexpr float BASE = W8 ? 0.0f : MM::BASE;
     f32x4 acc[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[b] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -497,7 +497,7 @@ __global__ __launch_bounds__(64 * kNzMaxWaves) void w4nz_decode(WqbmmArgs p, int
                 for (int j = u * JS; j < (u + 1) * JS; ++j) {
                     if constexpr (W8)
                         ag = MM::mma(xk[j],
-                                     nz8_operand<DT>(wk[b][j >> 1][2 * (j & 1)], wk[b][j >> 1][2 * (j & 1) + 1]), ag);
+                                     i8_operand<DT>(wk[b][j >> 1][2 * (j & 1)], wk[b][j >> 1][2 * (j & 1) + 1]), ag);
                     else
                         ag = MM::mma(xk[j], nz_operand<MM::MAGIC>(wk[b][0][j]), ag);
                 }

@@ -6,6 +6,7 @@ over at most 128 rows before the scale and the base's share, base * sum x, come 
 by at most u = 2^-24 * (base + max|w|) * sum of |x| over 128 rows.  A fold has 8 of them (four MFMAs for the products,
 four for the sum of x) and the K / 128 folds' errors add up as a random walk, so the rms error stays below
 8 * sqrt(K / 128) * u with a margin of about five; raw sums over all of K grow K / 128 times as large and miss it.
+int8 operands need no base (small weights show one: w + 128 would make the sums 64 times as large).
 """
 import math
 
@@ -55,4 +56,19 @@ def _rms_and_bar(ops, int4, layout, M, N, K, group, dtype, base, top, plan):
 ])
 def test_int4_long_groups(ops, layout, M, K, group, dtype, base, plan):
     rms, bar = _rms_and_bar(ops, True, layout, M, 272, K, group, dtype, base, 7, plan)
+    assert rms <= bar, (rms, bar)
+
+
+@pytest.mark.parametrize("layout,M,K,group,dtype,plan", [
+    ("nz", 100, 8192, 0, torch.float16, "nz_mid=1"),
+    ("nk", 40, 8192, 128, torch.bfloat16, "nz_mid=2"),
+    ("kn", 70, 64 * 65, 0, torch.float16, "nz_mid=1"),
+    ("nz", 200, 64 * 20, 64 * 5, torch.bfloat16, "nz_mid=1"),  # folds of four steps and one
+    ("nz", 16, 4096, 0, torch.float16, ""),                    # the decode kernel, even form
+    ("nz", 3, 64 * 65, 0, torch.bfloat16, ""),                 # its ragged form
+    ("nk", 9, 128 * 43, 128, torch.float16, ""),
+    ("nk", 40, 128 * 107, 0, torch.float16, "nz_mid=0"),
+])
+def test_int8_has_no_base(ops, layout, M, K, group, dtype, plan):
+    rms, bar = _rms_and_bar(ops, False, layout, M, 272, K, group, dtype, 0, 2, plan)
     assert rms <= bar, (rms, bar)
