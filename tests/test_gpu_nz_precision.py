@@ -1,12 +1,14 @@
 """fp32-level error of the weight-quant kernels on NZ and [N, K] weights, on the GPU.
 
-Rows of x come in equal pairs and rows of w in pairs of opposite sign, so every exact output is 0 and the output is
+Columns k and k + 32 of x are equal and rows k and k + 32 of w opposite (in every 64), so every exact output is 0 and the output is
 the error of the kernel's 32-bit sums alone (no 16-bit rounding hides it).  The kernels may sum x * (w + base) raw
 over at most 128 rows before the scale and the base's share, base * sum x, come off: one rounding of such a sum errs
 by at most u = 2^-24 * (base + max|w|) * sum of |x| over 128 rows.  A fold has 8 of them (four MFMAs for the products,
 four for the sum of x) and the K / 128 folds' errors add up as a random walk, so the rms error stays below
 8 * sqrt(K / 128) * u with a margin of about five; raw sums over all of K grow K / 128 times as large and miss it.
-int8 operands need no base (small weights show one: w + 128 would make the sums 64 times as large).
+int8 operands need no base: what 32 rows add the next 32 take off, so the sums stay below 32 rows' |w * x| and each
+MFMA errs by less than u0 = 2^-24 * max|w| * sum of |x| over 32 rows, K / 32 of them as a random walk.  With weights
+this small a base of 128 makes the sums 64 times as large.
 """
 import math
 
@@ -29,9 +31,10 @@ def ops():
 def _rms_and_bar(ops, int4, layout, M, N, K, group, dtype, base, top, plan):
     print(f"[case] int4={int4} {layout} M={M} N={N} K={K} G={group} {dtype} plan={plan!r}", flush=True)
     g = torch.Generator().manual_seed(M + K)
-    x = (0.5 + torch.rand((M, K // 2), generator=g)).to(dtype).repeat_interleave(2, 1)
-    w = torch.randint(-top, top + 1, (K // 2, N), generator=g, dtype=torch.int8).repeat_interleave(2, 0)
-    w[1::2] *= -1
+    x = torch.randn((M, K // 64, 1, 32), generator=g).abs().to(dtype)
+    x = x.expand(M, K // 64, 2, 32).reshape(M, K)
+    w = torch.randint(-top, top + 1, (K // 64, 1, 32, N), generator=g, dtype=torch.int8)
+    w = torch.cat([w, -w], 1).reshape(K, N)
     if layout == "nk":
         wd = w.t().contiguous().to(DEV).t()
     else:
@@ -41,8 +44,11 @@ def _rms_and_bar(ops, int4, layout, M, N, K, group, dtype, base, top, plan):
     ops.debug_set_plan(plan)
     out = ops.npu_weight_quant_batchmatmul(x.to(DEV), wd, s, antiquant_group_size=group)
     ops.debug_set_plan("")
-    u = 2.0 ** -24 * (base + top) * 128 * x.float().mean().item()
-    return out.float().square().mean().sqrt().item(), 8 * math.sqrt(K / 128) * u
+    rows, roundings = (128, 8) if base else (32, 1)
+    u = 2.0 ** -24 * (base + top) * rows * x.float().mean().item()
+    rms, bar = out.float().square().mean().sqrt().item(), roundings * math.sqrt(K / rows) * u
+    print(f"rms {rms:.3g} bar {bar:.3g}", flush=True)
+    return rms, bar
 
 
 @pytest.mark.parametrize("layout,M,K,group,dtype,base,plan", [
