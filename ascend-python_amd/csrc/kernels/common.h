@@ -510,6 +510,8 @@ size_t w4_nz_workspace(const WqbmmArgs& args, bool stream_k = true);
 size_t w4_cast_nz_workspace(const WqbmmArgs& args, bool stream_k = true);
 bool launch_w4_cast_nz(const WqbmmArgs& args, void* workspace, size_t ws_bytes, hipStream_t stream, hipError_t* err);
 hipError_t launch_w4_nz_bmm(const WqbmmArgs& args, void* workspace, size_t ws_bytes, hipStream_t stream);
+// One thread per output: any weight layout, shape and alignment, no workspace (w4a16_gemm.hip; args.group resolved).
+hipError_t launch_wq_generic(const WqbmmArgs& args, hipStream_t stream);
 // The mid-M kernel on NZ (int4, int8) and int8 [N, K] weights (nz_mid.hip; args.group resolved, not 0).
 double nz_mid_estimate(const WqbmmArgs& args);  // us; negative where it does not take the call
 size_t nz_mid_workspace(const WqbmmArgs& args);

@@ -1323,8 +1323,10 @@ hipError_t launch_w4_nz_bmm(const WqbmmArgs& p, void* workspace, size_t ws_bytes
     const int nd_dtype = w8 ? QK_I8 : QK_I32;
     const size_t nd_bytes = round256(nd_weight_bytes(p));
     const size_t rest = weight_quant_bmm_workspace(p.M, p.N, p.K, nd_dtype, p.group, true);
+    // The size query plans for 16-byte aligned operands, so a call whose operands are not, on a shape that a kernel
+    // above takes when they are, has no room for the ND weight: the general kernel reads the NZ weight as it is.
     if (!workspace || ws_bytes < QK_SPLIT_COUNTER_BYTES + nd_bytes + rest || (uintptr_t)workspace % 256 != 0)
-        return hipErrorInvalidValue;
+        return launch_wq_generic(p, stream);
     char* ws = static_cast<char*>(workspace);
     void* nd = ws + QK_SPLIT_COUNTER_BYTES;
     hipError_t e;

@@ -1354,7 +1354,29 @@ __global__ __launch_bounds__(pd::NT) void w4_dma(WqbmmArgs p, int tiles_m, int t
     }
 }
 
-// Any shape: one thread per output, fp32 sums per group then the same
+// Element (k, n) of the weight in any of its layouts.
+__device__ __forceinline__ int weight_at(const WqbmmArgs& p, int64_t k, int64_t n) {
+    const uint32_t* w4 = static_cast<const uint32_t*>(p.w);
+    const int8_t* w8 = static_cast<const int8_t*>(p.w);
+    uint32_t nib;
+    switch (p.w_dtype) {
+    case QK_I32: nib = w4[k * (p.N >> 3) + (n >> 3)] >> (4 * (n & 7)); break;
+    case QK_I4_NZ: {  // block (n / 16, k / 128), lane n % 16 + 16 * (8-row chunk % 4), word chunk / 4
+        const int c = (int)(k & 127) >> 3, i = (int)k & 7;
+        nib = w4[(((n >> 4) * (p.K >> 7) + (k >> 7)) * 64 + (n & 15) + 16 * (c & 3)) * 4 + (c >> 2)] >>
+              (4 * ((i & 1) ? 4 + (i >> 1) : (i >> 1)));
+        break;
+    }
+    case QK_I8_NZ:  // block (n / 16, k / 64), lane n % 16 + 16 * (16-row chunk)
+        return w8[(((n >> 4) * (p.K >> 6) + (k >> 6)) * 64 + (n & 15) + 16 * ((k & 63) >> 4)) * 16 + (k & 15)];
+    case QK_I8_NK: return w8[n * p.K + k];
+    default: return w8[k * p.N + n];
+    }
+    nib &= 0xfu;
+    return nib >= 8 ? (int)nib - 16 : (int)nib;
+}
+
+// Any shape, layout and alignment, no workspace: one thread per output, fp32 sums per group then the same
 // group-wise scale/offset algebra as the tiled kernels.
 __global__ __launch_bounds__(kThreads) void wq_generic(WqbmmArgs p) {
     const int64_t total = p.M * p.N;
@@ -1370,15 +1392,7 @@ __global__ __launch_bounds__(kThreads) void wq_generic(WqbmmArgs p) {
             const int64_t kend = (g + 1) * G < p.K ? (g + 1) * G : p.K;
             for (int64_t k = g * G; k < kend; ++k) {
                 const float xv = load_half_bits(X[m * p.K + k], p.x_dtype);
-                int wv;
-                if (p.w_dtype == QK_I32) {
-                    const uint32_t word = static_cast<const uint32_t*>(p.w)[k * (p.N >> 3) + (n >> 3)];
-                    wv = (int)((word >> (4 * (n & 7))) & 0xfu);
-                    wv = wv >= 8 ? wv - 16 : wv;
-                } else {
-                    wv = static_cast<const int8_t*>(p.w)[k * p.N + n];
-                }
-                sw = __builtin_fmaf(xv, (float)wv, sw);
+                sw = __builtin_fmaf(xv, (float)weight_at(p, k, n), sw);
                 xs += xv;
             }
             const float s = load_half_bits(static_cast<const uint16_t*>(p.scale)[g * p.N + n], p.s_dtype);
@@ -1707,6 +1721,14 @@ hipError_t launch_reduce(const WqbmmArgs& p, int nsplit, const float* partial, h
 
 }  // namespace
 
+hipError_t launch_wq_generic(const WqbmmArgs& p, hipStream_t stream) {
+    const int64_t total = p.M * p.N;
+    int64_t blocks = (total + kThreads - 1) / kThreads;
+    if (blocks > 65536) blocks = 65536;
+    wq_generic<<<dim3((uint32_t)blocks), dim3(kThreads), 0, stream>>>(p);
+    return hipGetLastError();
+}
+
 hipError_t launch_w4_xsum(const WqbmmArgs& p, float* xsum, hipStream_t stream) {
     const int64_t sums = p.M * (p.K / p.group);
     if (p.group >= kXsumWaveGroup) {
@@ -1856,11 +1878,7 @@ hipError_t launch_weight_quant_bmm(const WqbmmArgs& a, void* workspace, size_t w
         return p.x_dtype == QK_BF16 ? launch_gemm_dt<QK_BF16>(p, gf, nullptr, stream)
                                     : launch_gemm_dt<QK_F16>(p, gf, nullptr, stream);
     }
-    const int64_t total = p.M * p.N;
-    int64_t blocks = (total + kThreads - 1) / kThreads;
-    if (blocks > 65536) blocks = 65536;
-    wq_generic<<<dim3((uint32_t)blocks), dim3(kThreads), 0, stream>>>(p);
-    return hipGetLastError();
+    return launch_wq_generic(p, stream);
 }
 
 hipError_t launch_int4_pack(const void* w, int w_dtype, int64_t K, int64_t N, int32_t* packed, hipStream_t stream) {

@@ -61,6 +61,10 @@ at::Tensor workspace_for(const at::Tensor& like, size_t bytes) {
     return at::empty({(int64_t)bytes}, like.options().dtype(at::kByte));
 }
 
+// t itself, or a copy of it where its data is not 16-byte aligned (a view at an odd offset): the kernels' whole-line
+// loads need that.
+at::Tensor aligned16(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0 ? t.clone() : t; }
+
 // Rows of an [..., K] operand: the product of the leading dims (also when K == 0).
 int64_t leading_rows(const at::Tensor& t) {
     int64_t m = 1;
@@ -298,9 +302,8 @@ QmmPlan quant_matmul_plan(const at::Tensor& x1, const at::Tensor& x2, const at::
 at::Tensor quant_matmul_nz(const QmmPlan& pl, at::Tensor x1, const at::Tensor& x2_in, const at::Tensor& scale_in,
                            const std::optional<at::Tensor>& offset, const std::optional<at::Tensor>& pertoken_scale,
                            const std::optional<at::Tensor>& bias, at::Tensor out) {
-    if (reinterpret_cast<uintptr_t>(x1.data_ptr()) % 16 != 0) x1 = x1.clone();
-    auto x2 = x2_in.contiguous();
-    if (reinterpret_cast<uintptr_t>(x2.data_ptr()) % 16 != 0) x2 = x2.clone();
+    x1 = aligned16(x1);
+    auto x2 = aligned16(x2_in.contiguous());
     auto scale = scale_in.scalar_type() == at::kFloat ? scale_in.contiguous() : scale_in.to(at::kFloat);
     at::Tensor off, pt, b;
     if (offset.has_value()) off = offset->contiguous();
@@ -467,16 +470,17 @@ at::Tensor npu_weight_quant_batchmatmul(const at::Tensor& x_in, const at::Tensor
     const c10::DeviceGuard guard(x_in.device());
     auto out = at::empty(pl.out_shape, x_in.options());
     if (out.numel() == 0) return out;
-    auto x = x_in.contiguous();
+    auto x = aligned16(x_in.contiguous());
     // the weight is read where it lies: NZ blocks, [K, N] rows, or an int8 [N, K] tensor seen transposed; any
     // other strides are made contiguous (per slice of a batch, the last two dims decide)
     const bool nk = !pl.nz && int8_nk_view(weight_in, pl.K, pl.N);
     const int64_t d = weight_in.dim();
     const bool rows = !pl.nz && weight_in.stride(d - 1) == 1 && weight_in.stride(d - 2) == weight_in.size(d - 1);
     auto w = (pl.nz || nk || rows) ? weight_in : weight_in.contiguous();
-    auto sc = antiquant_scale.contiguous();
+    if (pl.nz || nk) w = aligned16(w);  // row-major weights have kernels for any alignment
+    auto sc = aligned16(antiquant_scale.contiguous());
     at::Tensor off, b;
-    if (antiquant_offset.has_value()) off = antiquant_offset->contiguous();
+    if (antiquant_offset.has_value()) off = aligned16(antiquant_offset->contiguous());
     if (bias.has_value()) b = bias->contiguous();
     const int wdt = pl.nz ? (pl.int4 ? QK_I4_NZ : QK_I8_NZ) : (pl.int4 ? QK_I32 : (nk ? QK_I8_NK : QK_I8));
     size_t ws_bytes = 0;

@@ -214,6 +214,10 @@ int qk_weight_quant_bmm_workspace_size(int64_t M, int64_t N, int64_t K, int weig
  * bias: [N] or NULL.  out: [M,N] of out_dtype (fp16/bf16).
  * out = sum_k x[m,k] * (w[k,n] + offset[g,n]) * scale[g,n] + bias[n], g = k/group,
  * with fp32 accumulation; the dequantized weight is never rounded to 16 bits.
+ * The pointers need no more than their element's alignment; x, weight (NZ and
+ * [N, K]), antiquant_scale, antiquant_offset and out that are not 16-byte
+ * aligned may run a general kernel, at a fraction of the speed (the torch op
+ * copies such operands first).
  */
 int qk_weight_quant_bmm(const void* x, int x_dtype,
                         const void* weight, int weight_dtype,
