@@ -1280,11 +1280,9 @@ bool nz_mid_wanted(const WqbmmArgs& p) {
 
 size_t w4_nz_workspace(const WqbmmArgs& p, bool stream_k) {
     if (stream_k && nz_mid_wanted(p)) return nz_mid_workspace(p);  // a launch given less runs the kernels below
-    // the decode kernel needs none; with 64-row groups the query keeps reporting the room of the ND form
-    const NzPlan z = plan_override().w4nz_off ? NzPlan{} : nz_plan(p);
-    if (z.ok && z.sub == 1) return 0;
-    if (!z.ok && nz_chunks_ok(p)) return 0;
-    if (!plan_override().w4nz_off && nzg_plan(p).ok) return nzg_workspace(p, stream_k);
+    const bool off = plan_override().w4nz_off;
+    if ((!off && nz_plan(p).ok) || nz_chunks_ok(p)) return 0;  // the decode kernel needs none
+    if (!off && nzg_plan(p).ok) return nzg_workspace(p, stream_k);
     const int nd_dtype = p.w_dtype == QK_I4_NZ ? QK_I32 : QK_I8;
     return QK_SPLIT_COUNTER_BYTES + round256(nd_weight_bytes(p)) +
            weight_quant_bmm_workspace(p.M, p.N, p.K, nd_dtype, p.group, true);
