@@ -661,6 +661,12 @@ __host__ __device__ __forceinline__ int64_t dma_k_len(int64_t K, int nsplit) {
     return ((K + ring - 1) / ring + nsplit - 1) / nsplit * ring;
 }
 
+// of `nsplit` such ranges, those that have rows of K: 5120 in eight splits of 640 runs as seven of 768 (the last 512)
+__host__ __device__ __forceinline__ int dma_splits(int64_t K, int nsplit) {
+    const int64_t len = dma_k_len(K, nsplit);
+    return (int)((K + len - 1) / len);
+}
+
 // BMX = 128 (K splits only): 128-row tiles, so a shape with few 256-row tiles needs half the K splits (and half
 // the int32 partials) to fill the CUs.  Waves then own 32 x 128 (two row tiles), an A slot is 16 KB, and each
 // split stores its exact sums in the MFMA output layout, one whole KB per store instruction:
@@ -2194,7 +2200,8 @@ hipError_t launch_quant_matmul(const QmmArgs& p, void* workspace, size_t ws_byte
     if (big_ok && bp.ragged && bp.nsplit > 1 && !big_dma_ok(p, b_kn, bp.nsplit)) big_ok = false;
     // a split of a ragged M runs only on the direct-to-LDS kernel; otherwise the register-staged kernel runs
     // the shape unsplit (the planned workspace is then unused)
-    if (big_ok && bp.nsplit > 1 && p.M % big::BM != 0 && !big_dma_ok(p, b_kn, bp.nsplit)) bp.nsplit = 1;
+    if (big_ok && bp.nsplit > 1 && big_dma_ok(p, b_kn, bp.nsplit)) bp.nsplit = dma_splits(p.K, bp.nsplit);
+    else if (big_ok && bp.nsplit > 1 && p.M % big::BM != 0) bp.nsplit = 1;
     if (big_ok && bp.nsplit > 1) {
         // splits need whole aligned tiles and the workspace; otherwise the tiled kernels take the shape
         const size_t need = QK_SPLIT_COUNTER_BYTES + (size_t)bp.nsplit * p.M * p.N * sizeof(int32_t);
@@ -2269,6 +2276,12 @@ hipError_t launch_nzd(const QmmArgs& p, const NzdPlan& z, hipStream_t stream) {
 // NZ weight may be ragged)
 bool nz_dma_ok(const BigPlan& b) { return plan_override().qmm_dma && b.ok; }
 
+BigPlan nz_big_plan(int64_t M, int64_t N, int64_t K) {
+    BigPlan b = big_plan(M, N, K);
+    if (b.ok && b.nsplit > 1) b.nsplit = dma_splits(K, b.nsplit);
+    return b;
+}
+
 template <int OUT>
 hipError_t launch_dma_nz(const QmmArgs& p, const BigPlan& b, int32_t* partial, hipStream_t stream) {
     if (b.bm != 256) return hipErrorInvalidValue;  // 256-row tiles: tiles_m counts them
@@ -2289,7 +2302,7 @@ size_t quant_matmul_nz_workspace(int64_t M, int64_t N, int64_t K) {
         const int ns = small_split(M, N, K, mid_plan(M, N, K, false), kMidHbmNz);
         return ns ? big_split_workspace(small_split_plan(M, N, ns), M, N) : 0;
     }
-    const BigPlan b = big_plan(M, N, K);
+    const BigPlan b = nz_big_plan(M, N, K);
     if (nz_dma_ok(b)) return b.nsplit > 1 ? big_split_workspace(b, M, N) : 0;
     return round_up256((size_t)K * (size_t)N) + quant_matmul_workspace(M, N, K);
 }
@@ -2313,7 +2326,7 @@ hipError_t launch_quant_matmul_nz(const QmmArgs& p, void* workspace, size_t ws_b
         }
         return launch_mid<kLayNZ>(p, mp, nullptr, nullptr, stream);
     }
-    const BigPlan b = big_plan(p.M, p.N, p.K);
+    const BigPlan b = nz_big_plan(p.M, p.N, p.K);
     if (nz_dma_ok(b)) {
         if (b.nsplit == 1) {
             switch (p.epi.out_dtype) {

@@ -44,6 +44,8 @@ SHAPES = [
     (129, 8272, 2064),
     (700, 272, 5504),
     (257, 49184, 320),   # 2 x 193 whole tiles: no split
+    (300, 1536, 5120),   # eight even K ranges of no whole rings: seven run
+    (512, 1536, 5120),
 ]
 
 

@@ -77,6 +77,9 @@ def test_w8a8_split_plan_workspace_sizes():
         assert ws.value == ctr + 8 * 128 * 4096 * 4
         assert L.qk_quant_matmul_nz_workspace_size(128, 11008, 4096, BF16, ctypes.byref(ws)) == 0
         assert ws.value == 0
+        # eight even ranges of K = 5120 are no whole 256-row rings: seven ranges of at most 768 rows hold all of K
+        assert L.qk_quant_matmul_nz_workspace_size(300, 1536, 5120, BF16, ctypes.byref(ws)) == 0
+        assert ws.value == ctr + 7 * 300 * 1536 * 4
         q.debug_set_plan("qmm_small=0")
         assert L.qk_quant_matmul_workspace_size(128, 11008, 4096, BF16, ctypes.byref(ws)) == 0
         assert ws.value == 0
