@@ -513,9 +513,17 @@ hipError_t launch_w4_nz_bmm(const WqbmmArgs& args, void* workspace, size_t ws_by
 // One thread per output: any weight layout, shape and alignment, no workspace (w4a16_gemm.hip; args.group resolved).
 hipError_t launch_wq_generic(const WqbmmArgs& args, hipStream_t stream);
 // The mid-M kernel on NZ (int4, int8) and int8 [N, K] weights (nz_mid.hip; args.group resolved, not 0).
-double nz_mid_estimate(const WqbmmArgs& args);  // us; negative where it does not take the call
-size_t nz_mid_workspace(const WqbmmArgs& args);
-hipError_t launch_nz_mid(const WqbmmArgs& args, void* workspace, size_t ws_bytes, hipStream_t stream);
+// The plan weighs up to 48 tilings (0.2 us of host time): one per query or launch, handed on.
+struct NzMidPlan {
+    bool ok = false;  // takes the call
+    bool half = false;
+    int tm = 0, tiles_m = 0, tiles_n = 0, nsplit = 1;
+    double us = 0;  // estimate
+};
+NzMidPlan nz_mid_plan(const WqbmmArgs& args);
+size_t nz_mid_workspace(const NzMidPlan& plan);
+hipError_t launch_nz_mid(const WqbmmArgs& args, const NzMidPlan& plan, void* workspace, size_t ws_bytes,
+                         hipStream_t stream);
 
 // Static quantization (static_quant.hip): x [outer][C][inner] (fp32/fp16/bf16) -> q (int8/uint8/int32);
 // scales == nullptr: per tensor with scale0 / zp0.

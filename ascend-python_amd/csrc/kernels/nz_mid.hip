@@ -381,15 +381,10 @@ __global__ __launch_bounds__(256) void nz_mid_reduce(WqbmmArgs p, int tm_frags, 
     }
 }
 
-struct Plan {
-    bool ok = false;
-    int tm = 0, tiles_m = 0, tiles_n = 0, nsplit = 1;
-    bool half = false;
-    double us = 0;  // estimate
-};
+}  // namespace
 
-Plan mid_plan(const WqbmmArgs& p) {
-    Plan z;
+NzMidPlan nz_mid_plan(const WqbmmArgs& p) {
+    NzMidPlan z;
     const int64_t G = p.group == 0 ? p.K : p.group;
     const bool w8 = p.w_dtype == QK_I8_NZ || p.w_dtype == QK_I8_NK;
     const int ks = nm::ksw(w8);
@@ -404,7 +399,7 @@ Plan mid_plan(const WqbmmArgs& p) {
     if (((uintptr_t)p.x | (uintptr_t)p.w | (uintptr_t)p.scale | (uintptr_t)p.out |
          (uintptr_t)(p.offset ? p.offset : p.scale)) % 16 != 0)
         return z;
-    const int64_t S = p.K / ks;
+    const int S = (int)(p.K / ks);
     z.tiles_n = (int)((p.N + 255) / 256);
     if ((p.M + 31) / 32 * z.tiles_n >= ((int64_t)1 << 20)) return z;
     // Row tiles of at most 96 rows (64 with half-step groups), all of one height, and the K split: the pair with the
@@ -412,11 +407,11 @@ Plan mid_plan(const WqbmmArgs& p) {
     // / 1.58 with 2 / 4 / 6 row tiles of 16; int8, 64 rows: 0.82 / 0.96): rounds of workgroups x steps, about 5 of
     // launch, first loads and epilogue, and for a split another launch and the partials written and read.
     const int most = z.half ? 4 : 6;
-    const int64_t t16 = (p.M + 15) / 16, tm_lo = (t16 + most - 1) / most;
-    for (int64_t tm = tm_lo; tm <= tm_lo + 2 && tm <= t16; ++tm) {
-        const int h = (int)std::max<int64_t>(2, (t16 + tm - 1) / tm);
+    const int t16 = (int)((p.M + 15) / 16), tm_lo = (t16 + most - 1) / most;
+    for (int tm = tm_lo; tm <= tm_lo + 2 && tm <= t16; ++tm) {
+        const int h = std::max(2, (t16 + tm - 1) / tm);
         const double step = w8 ? 0.72 + 0.045 * h : 0.65 + 0.155 * h;
-        const int64_t tiles = tm * z.tiles_n;
+        const int tiles = tm * z.tiles_n;  // below 2^22
         for (int ns = 1; ns <= 16 && ns <= S; ++ns) {
             if (ov.nz_mid > 0 && ov.nz_mid < 17 && ns != ov.nz_mid) continue;
             const double part = (double)ns * (double)tiles * h * 16 * 256 * 4;
@@ -426,7 +421,7 @@ Plan mid_plan(const WqbmmArgs& p) {
             if (z.ok && t >= z.us) continue;
             z.us = t;
             z.tm = h;
-            z.tiles_m = (int)tm;
+            z.tiles_m = tm;
             z.nsplit = ns;
             z.ok = true;
         }
@@ -434,8 +429,10 @@ Plan mid_plan(const WqbmmArgs& p) {
     return z;
 }
 
+namespace {
+
 template <int DT, int TM, bool W8>
-void launch_mode(const WqbmmArgs& p, const Plan& z, float* part, hipStream_t stream) {
+void launch_mode(const WqbmmArgs& p, const NzMidPlan& z, float* part, hipStream_t stream) {
     const bool nk = p.w_dtype == QK_I8_NK;
     const uint32_t wblk = nk ? 16u * (uint32_t)p.K : (uint32_t)(p.K / nm::ksw(W8)) * 1024u, wstep = nk ? 64u : 1024u;
     const dim3 grid((uint32_t)(z.tiles_m * z.tiles_n * z.nsplit)), block(nm::NT);
@@ -448,7 +445,7 @@ void launch_mode(const WqbmmArgs& p, const Plan& z, float* part, hipStream_t str
 }
 
 template <int DT, bool W8>
-void launch_tm(const WqbmmArgs& p, const Plan& z, float* part, hipStream_t stream) {
+void launch_tm(const WqbmmArgs& p, const NzMidPlan& z, float* part, hipStream_t stream) {
     switch (z.tm) {
     case 2: launch_mode<DT, 2, W8>(p, z, part, stream); break;
     case 3: launch_mode<DT, 3, W8>(p, z, part, stream); break;
@@ -461,23 +458,16 @@ void launch_tm(const WqbmmArgs& p, const Plan& z, float* part, hipStream_t strea
 }  // namespace
 
 // [split counters, unused][partials fp32 [split][tile][rows x 256]]
-size_t nz_mid_workspace(const WqbmmArgs& p) {
-    const Plan z = mid_plan(p);
+size_t nz_mid_workspace(const NzMidPlan& z) {
     if (!z.ok || z.nsplit == 1) return 0;
     return QK_SPLIT_COUNTER_BYTES + (size_t)z.nsplit * z.tiles_m * z.tiles_n * z.tm * 16 * 256 * sizeof(float);
 }
 
-double nz_mid_estimate(const WqbmmArgs& p) {
-    const Plan z = mid_plan(p);
-    return z.ok ? z.us : -1.0;
-}
-
-hipError_t launch_nz_mid(const WqbmmArgs& p, void* workspace, size_t ws_bytes, hipStream_t stream) {
-    const Plan z = mid_plan(p);
+hipError_t launch_nz_mid(const WqbmmArgs& p, const NzMidPlan& z, void* workspace, size_t ws_bytes, hipStream_t stream) {
     if (!z.ok) return hipErrorInvalidValue;
     float* part = nullptr;
     if (z.nsplit > 1) {
-        if (!workspace || ws_bytes < nz_mid_workspace(p) || (uintptr_t)workspace % 16 != 0) return hipErrorInvalidValue;
+        if (!workspace || ws_bytes < nz_mid_workspace(z) || (uintptr_t)workspace % 16 != 0) return hipErrorInvalidValue;
         part = reinterpret_cast<float*>(static_cast<char*>(workspace) + QK_SPLIT_COUNTER_BYTES);
     }
     const bool w8 = p.w_dtype != QK_I4_NZ;

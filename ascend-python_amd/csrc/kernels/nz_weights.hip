@@ -1201,7 +1201,7 @@ hipError_t launch_w8_nz_cast(const int8_t* src, bool to_nz, int64_t K, int64_t N
 }
 
 // NZ weights (int4 QK_I4_NZ, int8 QK_I8_NZ): the decode kernel where it applies (no workspace), the mid-M kernel
-// or the prefill kernel (nz_mid_wanted weighs them);
+// or the prefill kernel (nz_mid_ahead weighs them);
 // otherwise the weight is unpacked into the workspace and the row-major kernels run on it:
 // [QK_SPLIT_COUNTER_BYTES, unused][ND weight][row-major call's workspace].
 // An int8 [N, K] weight (QK_I8_NK) takes the same decode kernel (reading it in place) or is transposed into the
@@ -1249,12 +1249,8 @@ double nz_decode_estimate(const WqbmmArgs& p) {
     return (double)(((int64_t)z.nwg * z.nrb + 255) / 256) * z.nit * (1.35 + c * z.nb) + 2.0;
 }
 
-bool nz_mid_wanted(const WqbmmArgs& p) {
-    const int ov = plan_override().nz_mid;  // debug override: never, or wherever it can
-    if (ov == 0 || p.M <= 16) return false;
-    const double t = nz_mid_estimate(p);
-    if (t < 0) return false;
-    if (ov > 0) return true;
+bool nz_mid_ahead(const WqbmmArgs& p, double t) {  // t: its estimate
+    if (plan_override().nz_mid > 0) return true;  // debug override: wherever it can
     if (p.M <= kNzChunkRows) {
         const double d = nz_decode_estimate(p);
         return d < 0 || t < d;
@@ -1278,8 +1274,16 @@ bool nz_mid_wanted(const WqbmmArgs& p) {
     return t < rounds * steps * (w8 ? 1.15 : 2.05) + 8.0 + casts;
 }
 
+// The mid-M kernel's plan where it is taken, else one that is not ok.
+NzMidPlan nz_mid_wanted(const WqbmmArgs& p) {
+    if (plan_override().nz_mid == 0 || p.M <= 16) return NzMidPlan{};
+    const NzMidPlan z = nz_mid_plan(p);
+    return z.ok && nz_mid_ahead(p, z.us) ? z : NzMidPlan{};
+}
+
 size_t w4_nz_workspace(const WqbmmArgs& p, bool stream_k) {
-    if (stream_k && nz_mid_wanted(p)) return nz_mid_workspace(p);  // a launch given less runs the kernels below
+    if (stream_k)  // a launch given less runs the kernels below
+        if (const NzMidPlan mid = nz_mid_wanted(p); mid.ok) return nz_mid_workspace(mid);
     const bool off = plan_override().w4nz_off;
     if ((!off && nz_plan(p).ok) || nz_chunks_ok(p)) return 0;  // the decode kernel needs none
     if (!off && nzg_plan(p).ok) return nzg_workspace(p, stream_k);
@@ -1289,8 +1293,10 @@ size_t w4_nz_workspace(const WqbmmArgs& p, bool stream_k) {
 }
 
 hipError_t launch_w4_nz_bmm(const WqbmmArgs& p, void* workspace, size_t ws_bytes, hipStream_t stream) {
-    if (nz_mid_wanted(p) && (nz_mid_workspace(p) == 0 || (workspace && ws_bytes >= nz_mid_workspace(p))))
-        return launch_nz_mid(p, workspace, ws_bytes, stream);
+    if (const NzMidPlan mid = nz_mid_wanted(p); mid.ok) {
+        const size_t need = nz_mid_workspace(mid);
+        if (need == 0 || (workspace && ws_bytes >= need)) return launch_nz_mid(p, mid, workspace, ws_bytes, stream);
+    }
     const NzPlan z = plan_override().w4nz_off ? NzPlan{} : nz_plan(p);
     if (z.ok)
         return p.x_dtype == QK_BF16 ? launch_nz_dt<QK_BF16>(p, z, stream) : launch_nz_dt<QK_F16>(p, z, stream);
@@ -1376,28 +1382,45 @@ bool cast_nz_decode(const WqbmmArgs& p) {
 // / 127.7 against 34.2 / 52.4 / 76.0), the register-staged prefill kernel at 1.75 us per 64-row step and round of its
 // 256 x 128 tiles (N = 32000, K = 4096, M = 20-100 114-119 us against 53-80; it also takes every K of no whole 256
 // rows: K = 11008 92 us against 26-49).
-bool cast_nz_mid(const WqbmmArgs& q) {
-    if (q.w_dtype == QK_I8_NZ) return q.M > 32 && nz_mid_wanted(q);
+struct CastNzPlan {
+    bool ok = false;
+    NzMidPlan mid;  // not ok: the decode kernel
+    size_t bytes = 0;  // [counters][NZ weight][the mid-M kernel's workspace]
+};
+
+bool cast_nz_mid_ahead(const WqbmmArgs& q, const NzMidPlan& mid) {
+    if (q.w_dtype == QK_I8_NZ) return mid.ok && q.M > 32;
     if (plan_override().nz_mid == 0) return false;
-    const bool mid = nz_mid_wanted(q);
-    if (mid && (q.M > 256 || plan_override().nz_mid > 0)) return true;
-    if (q.M <= 16 || (!mid && !(q.M <= kNzChunkRows && nz_plan(q).ok))) return false;
+    if (mid.ok && (q.M > 256 || plan_override().nz_mid > 0)) return true;
+    if (q.M <= 16 || (!mid.ok && !(q.M <= kNzChunkRows && nz_plan(q).ok))) return false;
     const double mb = 0.5e-6 * (double)(q.K * q.N);
     const int64_t tiles = (q.M + 255) / 256 * ((q.N + 127) / 128);
     const bool blocks = q.K % 256 == 0 && tiles < 128;
     const double rows = blocks ? 8.0 + 0.22 * mb * (double)((q.M + 15) / 16)
                                : 1.75 * (double)(q.K / 64) * (double)((tiles + 255) / 256);
-    return (mid ? nz_mid_estimate(q) : nz_decode_estimate(q)) + 6.5 + 0.22 * mb < rows;
+    return (mid.ok ? mid.us : nz_decode_estimate(q)) + 6.5 + 0.22 * mb < rows;
+}
+
+CastNzPlan cast_nz_mid(const WqbmmArgs& q) {
+    CastNzPlan c;
+    c.mid = nz_mid_wanted(q);
+    c.ok = cast_nz_mid_ahead(q, c.mid);
+    c.bytes = round256(QK_SPLIT_COUNTER_BYTES + round256(nd_weight_bytes(q)) + nz_mid_workspace(c.mid));
+    return c;
+}
+
+bool cast_nz_off(const WqbmmArgs& p) {
+    const PlanOverride& ov = plan_override();
+    return !(p.w_dtype == QK_I32 || p.w_dtype == QK_I8) || ov.w4nz_off || ov.w4_gemm != 0;
 }
 
 size_t w4_cast_nz_workspace(const WqbmmArgs& p, bool stream_k) {
-    const PlanOverride& ov = plan_override();
-    if (!(p.w_dtype == QK_I32 || p.w_dtype == QK_I8) || ov.w4nz_off || ov.w4_gemm != 0) return 0;
+    if (cast_nz_off(p)) return 0;
     WqbmmArgs q = p;
     q.w = reinterpret_cast<const void*>((uintptr_t)256);  // the cast's destination: 256-byte aligned
     q.w_dtype = p.w_dtype == QK_I8 ? QK_I8_NZ : QK_I4_NZ;
-    if (stream_k && cast_nz_mid(q))  // [counters][NZ weight][the mid-M kernel's workspace]
-        return round256(QK_SPLIT_COUNTER_BYTES + round256(nd_weight_bytes(q)) + (nz_mid_wanted(q) ? nz_mid_workspace(q) : 0));
+    if (stream_k)
+        if (const CastNzPlan c = cast_nz_mid(q); c.ok) return c.bytes;
     if (cast_nz_decode(p)) return round256(QK_SPLIT_COUNTER_BYTES + round256(nd_weight_bytes(q)));
     if (p.M < cast_nz_min_m(p.w_dtype) || !nzg_plan(q).ok) return 0;
     return round256(QK_SPLIT_COUNTER_BYTES + round256(nd_weight_bytes(q)) +
@@ -1405,22 +1428,23 @@ size_t w4_cast_nz_workspace(const WqbmmArgs& p, bool stream_k) {
 }
 
 bool launch_w4_cast_nz(const WqbmmArgs& p, void* workspace, size_t ws_bytes, hipStream_t stream, hipError_t* err) {
-    const size_t full = w4_cast_nz_workspace(p, true), need = w4_cast_nz_workspace(p, false);
-    if (full == 0 || !workspace || (uintptr_t)workspace % 256 != 0) return false;
+    if (cast_nz_off(p) || !workspace || (uintptr_t)workspace % 256 != 0) return false;
     char* ws = static_cast<char*>(workspace);
     void* nz = ws + QK_SPLIT_COUNTER_BYTES;
     const bool w8 = p.w_dtype == QK_I8;
     WqbmmArgs q = p;
     q.w = nz;
     q.w_dtype = w8 ? QK_I8_NZ : QK_I4_NZ;
-    if (ws_bytes >= full && cast_nz_mid(q)) {
+    if (const CastNzPlan c = cast_nz_mid(q); c.ok && ws_bytes >= c.bytes) {  // with the call's own operands
         hipError_t e = w8 ? launch_w8_nz_cast(static_cast<const int8_t*>(p.w), true, p.K, p.N, static_cast<int8_t*>(nz), stream)
                           : launch_w4_nz_cast(static_cast<const int32_t*>(p.w), true, p.K, p.N, static_cast<int32_t*>(nz), stream);
         const size_t used = QK_SPLIT_COUNTER_BYTES + round256(nd_weight_bytes(q));
-        if (e == hipSuccess) e = launch_w4_nz_bmm(q, ws + used, ws_bytes - used, stream);
+        if (e == hipSuccess)
+            e = c.mid.ok ? launch_nz_mid(q, c.mid, ws + used, ws_bytes - used, stream) : launch_w4_nz_bmm(q, nullptr, 0, stream);
         *err = e;
         return true;
     }
+    const size_t need = w4_cast_nz_workspace(p, false);
     if (need == 0 || ws_bytes < need) return false;
     if (cast_nz_decode(p)) {
         if (!nz_decode_ok(q)) return false;  // with the call's own operands (their alignment)
