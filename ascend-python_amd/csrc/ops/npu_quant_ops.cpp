@@ -924,12 +924,13 @@ at::Tensor npu_quant_matmul_swiglu(const at::Tensor& x1_in, const at::Tensor& x2
     int64_t K = 0, I = 0;
     const auto shape = swiglu_matmul_check(x1_in, x2_in, scale_in, pertoken_scale, out_type, K, I);
     const c10::DeviceGuard guard(x1_in.device());
-    auto out = at::empty(shape, x1_in.options().dtype(out_type));
-    if (out.numel() == 0) return out;
+    auto empty = [&] { return at::empty(shape, x1_in.options().dtype(out_type)); };
+    if (leading_rows(x1_in) * I == 0) return empty();
     const bool nz = is_w8_nz(x2_in);
-    auto x1 = x1_in.contiguous();
     const bool kn = !nz && x2_in.stride(1) == 1 && x2_in.stride(0) >= 2 * I;
-    if ((nz || kn) && !swiglu_chain(x1)) {
+    if ((nz || kn) && !swiglu_chain(x1_in)) {
+        auto x1 = x1_in.contiguous();
+        auto out = empty();
         auto scale = scale_in.scalar_type() == at::kFloat ? scale_in.contiguous() : scale_in.to(at::kFloat);
         at::Tensor pt;
         if (pertoken_scale.has_value()) pt = pertoken_scale->contiguous();
@@ -958,13 +959,16 @@ std::tuple<at::Tensor, at::Tensor> npu_quant_matmul_swiglu_quant(const at::Tenso
     int64_t K = 0, I = 0;
     const auto shape = swiglu_matmul_check(x1_in, x2_in, scale_in, pertoken_scale, h_type, K, I);
     const c10::DeviceGuard guard(x1_in.device());
-    auto q = at::empty(shape, x1_in.options().dtype(at::kChar));
-    auto qs = at::empty(at::IntArrayRef(shape).slice(0, shape.size() - 1), x1_in.options().dtype(at::kFloat));
-    if (q.numel() == 0) return {q, qs};
+    auto empty = [&]() -> std::tuple<at::Tensor, at::Tensor> {
+        return {at::empty(shape, x1_in.options().dtype(at::kChar)),
+                at::empty(at::IntArrayRef(shape).slice(0, shape.size() - 1), x1_in.options().dtype(at::kFloat))};
+    };
+    if (leading_rows(x1_in) * I == 0) return empty();
     const bool nz = is_w8_nz(x2_in);
-    auto x1 = x1_in.contiguous();
     const bool kn = !nz && x2_in.stride(1) == 1 && x2_in.stride(0) >= 2 * I;
-    if ((nz || kn) && !swiglu_chain(x1)) {
+    if ((nz || kn) && !swiglu_chain(x1_in)) {
+        auto x1 = x1_in.contiguous();
+        auto [q, qs] = empty();
         auto scale = scale_in.scalar_type() == at::kFloat ? scale_in.contiguous() : scale_in.to(at::kFloat);
         at::Tensor pt;
         if (pertoken_scale.has_value()) pt = pertoken_scale->contiguous();
