@@ -31,7 +31,8 @@
 // non-temporal), folds group scale and offset into its accumulators per
 // superblock with the algebra of the row-major kernels,
 //   acc += s * sum_k x*(w + BASE) + s*(offset - BASE) * sum_k x
-// (int8 operands are the bytes' own values: BASE = 0), and the waves' sums are added through LDS in K order (deterministic).
+// (int8 operands are the bytes' own values, BASE = 0, but for one form), and the waves' sums are added through LDS in K order (deterministic).
+#include <algorithm>
 #include <atomic>
 
 #include "common.h"
@@ -460,7 +461,11 @@ __global__ __launch_bounds__(64 * kNzMaxWaves) void w4nz_decode(WqbmmArgs p, int
     for (int it = 0; it < PF; ++it) issue(it, it);
 
     const u32x4 ones = {MM::ONES, MM::ONES, MM::ONES, MM::ONES};
-    constexpr float BASE = W8 ? 0.0f : MM::BASE;
+    // Waves of one superblock leave LDS for two workgroups per CU, which also takes at most 64 registers each.  Three int8
+    // blocks of them stay with the prefill kernel's operands w + 128: the others' conversion takes 90 registers there
+    // (K = 2048, N = 11008, M = 40 13.2 us against 11.3), and w + 128 - 128 in place of it 12.4.
+    constexpr bool PLUS128 = W8 && NIT == 1 && NB == 3;
+    constexpr float BASE = PLUS128 ? 128.0f : W8 ? 0.0f : MM::BASE;
     f32x4 acc[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[b] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -495,10 +500,10 @@ __global__ __launch_bounds__(64 * kNzMaxWaves) void w4nz_decode(WqbmmArgs p, int
                 f32x4 ag = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int j = u * JS; j < (u + 1) * JS; ++j) {
-                    if constexpr (W8)
-                        ag = MM::mma(xk[j],
-                                     i8_operand<DT>(wk[b][j >> 1][2 * (j & 1)], wk[b][j >> 1][2 * (j & 1) + 1]), ag);
-                    else
+                    if constexpr (W8) {
+                        const uint32_t lo = wk[b][j >> 1][2 * (j & 1)], hi = wk[b][j >> 1][2 * (j & 1) + 1];
+                        ag = MM::mma(xk[j], PLUS128 ? nz8_operand<DT>(lo, hi) : i8_operand<DT>(lo, hi), ag);
+                    } else
                         ag = MM::mma(xk[j], nz_operand<MM::MAGIC>(wk[b][0][j]), ag);
                 }
                 const float sf = load_half_bits(srow[wave][sl][u * NT][16 * b + c], SDT);
