@@ -31,7 +31,8 @@
 // non-temporal), folds group scale and offset into its accumulators per
 // superblock with the algebra of the row-major kernels,
 //   acc += s * sum_k x*(w + BASE) + s*(offset - BASE) * sum_k x
-// (int8 operands are the bytes' own values, BASE = 0, but for one form), and the waves' sums are added through LDS in K order (deterministic).
+// (int8 operands are the bytes' own values, BASE = 0, but for one form), and the
+// waves' sums are added through LDS in K order (deterministic).
 #include <algorithm>
 #include <atomic>
 
@@ -1241,7 +1242,10 @@ bool nz_chunks_ok(const WqbmmArgs& p) {
 //   decode kernel: every CU runs one workgroup at a time, and each of the 16-row blocks reads the weight again, so
 //     rounds of workgroups x superblocks per wave x (1.35 + c per block), c = 0.35 int4, 0.8 int8 NZ, 1.3 [N, K]
 //     (N = 11008, K = 4096, M = 20 / 40 12.2 / 17.4 measured; K = 11008, N = 4096, M = 64 40.8; K = 28672, N = 8192,
-//     M = 60 102; [N, K], N = 11008, K = 4096, M = 23 23.4);
+//     M = 60 102; [N, K], N = 11008, K = 4096, M = 23 23.4).  Fewer than 192 workgroups along N leave each of them more
+//     of the bandwidth, down to half the time (0.6 on [N, K]; K = 5120, N = 1536, 96 of them, M = 32 / 64 int4 6.5 /
+//     11.4, int8 7.5 / 12.6, [N, K] 9.3 / 16.0, against 11.1 / 12.4, 13.0 / 14.2, 14.3 / 15.2); rounds of one superblock
+//     per wave overlap (int8, K = 2048, N = 3072, M = 128 in two chunks 14.2 against 17.0, [N, K] M = 77 11.5 / 15.4);
 //   prefill kernel: 2.05 per 128-row int4 step (1.15 per 64-row int8 step) of one round of 128 x 256 tiles, and about
 //     8 of its launches (N = 11008, K = 4096, M = 250 / 400 66.8 / 67.9 against 45.8 / 52.4; N = 28672, M = 250 69.0
 //     against 90.7); from a tile per CU on it is ahead (N = 11008, M = 900 / 2000 102.7 / 197.9 against 111.5 / 226.1).
@@ -1251,7 +1255,10 @@ double nz_decode_estimate(const WqbmmArgs& p) {
     const NzPlan z = nz_plan(p);
     if (!z.ok) return -1.0;
     const double c = p.w_dtype == QK_I4_NZ ? 0.35 : p.w_dtype == QK_I8_NZ ? 0.8 : 1.3;
-    return (double)(((int64_t)z.nwg * z.nrb + 255) / 256) * z.nit * (1.35 + c * z.nb) + 2.0;
+    const double least = p.w_dtype == QK_I8_NK ? 0.6 : 0.5;
+    const double narrow = z.sub == 2 ? 1.0 : std::min(1.0, std::max(least, z.nwg / 192.0));  // 64-row groups: not seen
+    const double rounds = (double)(((int64_t)z.nwg * z.nrb + 255) / 256) * (z.nit == 1 ? 0.8 : 1.0);
+    return rounds * z.nit * (1.35 + c * z.nb) * narrow + 2.0;
 }
 
 bool nz_mid_ahead(const WqbmmArgs& p, double t) {  // t: its estimate
@@ -1385,8 +1392,13 @@ bool cast_nz_decode(const WqbmmArgs& p) {
 // and the kernel are weighed against them: the 16-row-block decode kernel at 8 us and 0.22 per MB and row block (N =
 // 4096, K = 4096, M = 20 / 100 / 250 10.6 / 22.5 / 36.3 us against 19.2 / 25.1 / 29.5; N = 13696, K = 5120 29.2 / 62.5
 // / 127.7 against 34.2 / 52.4 / 76.0), the register-staged prefill kernel at 1.75 us per 64-row step and round of its
-// 256 x 128 tiles (N = 32000, K = 4096, M = 20-100 114-119 us against 53-80; it also takes every K of no whole 256
-// rows: K = 11008 92 us against 26-49).
+// 256 x 128 tiles, 1.55 on whole ones (N = 32000, K = 4096, M = 20-100 114-119 us against 53-80, M = 256 with 64-row
+// groups 99 against 131; it also takes every K of no whole 256 rows: K = 11008 92 us against 26-49).  Past 256 rows the
+// prefill kernel on the cast weight is what was weighed, and where that does not take the shape the row-major kernels
+// again: the block kernel without its K split (256 workgroups and more) gets by on about K / 128 * (0.6 + workgroups /
+// 512) (K = 2048, N = 3072, M = 400 / 600 24.3 / 25.2 against 27.3 / 30.8), with 64-row groups 1.4 times that (37
+// against 27 at K = 5120, N = 1536, M = 300); int8 the prefill kernel alone (K = 5120, N = 13696, M = 300 / 400
+// 135 / 135 against 115 / 167, one group over K).
 struct CastNzPlan {
     bool ok = false;
     NzMidPlan mid;  // not ok: the decode kernel
@@ -1394,15 +1406,21 @@ struct CastNzPlan {
 };
 
 bool cast_nz_mid_ahead(const WqbmmArgs& q, const NzMidPlan& mid) {
-    if (q.w_dtype == QK_I8_NZ) return mid.ok && q.M > 32;
-    if (plan_override().nz_mid == 0) return false;
-    if (mid.ok && (q.M > 256 || plan_override().nz_mid > 0)) return true;
-    if (q.M <= 16 || (!mid.ok && !(q.M <= kNzChunkRows && nz_plan(q).ok))) return false;
-    const double mb = 0.5e-6 * (double)(q.K * q.N);
-    const int64_t tiles = (q.M + 255) / 256 * ((q.N + 127) / 128);
-    const bool blocks = q.K % 256 == 0 && tiles < 128;
-    const double rows = blocks ? 8.0 + 0.22 * mb * (double)((q.M + 15) / 16)
-                               : 1.75 * (double)(q.K / 64) * (double)((tiles + 255) / 256);
+    const int ov = plan_override().nz_mid;
+    const bool w8 = q.w_dtype == QK_I8_NZ;
+    if (w8 ? !mid.ok || q.M <= 32 : ov == 0 || q.M <= 16 || (!mid.ok && !(q.M <= kNzChunkRows && nz_plan(q).ok)))
+        return false;
+    if (mid.ok && ov > 0) return true;
+    if (q.M > 256 ? nzg_plan(q).ok : w8) return true;
+    const double mb = (w8 ? 1e-6 : 0.5e-6) * (double)(q.K * q.N);
+    const int64_t tiles = (q.M + 255) / 256 * ((q.N + 127) / 128), rb = (q.M + 15) / 16;
+    double rows = (!w8 && q.M % 256 == 0 && q.N % 128 == 0 ? 1.55 : 1.75) * (double)(q.K / 64) * (double)((tiles + 255) / 256);
+    if (!w8 && q.K % 256 == 0 && tiles < 128) {  // the 16-row-block kernel, strips of 256 columns
+        rows = 8.0 + 0.22 * mb * (double)rb;
+        if (const int64_t wgs = (q.N + 255) / 256 * rb; q.M > 256 && wgs >= 256)
+            rows = std::min(rows, 2.0 + (double)q.K / 128.0 * (0.6 + (double)wgs / 512.0));
+        if (q.M > 256 && q.group == 64) rows *= 1.4;
+    }
     return (mid.ok ? mid.us : nz_decode_estimate(q)) + 6.5 + 0.22 * mb < rows;
 }
 

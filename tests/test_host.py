@@ -48,6 +48,28 @@ def test_debug_plan_override_parsing():
     q.debug_set_plan("")
 
 
+def test_mid_m_plan_sizes():
+    """Where the weight-quant mid-M kernel is taken its K splits report a workspace; where the kernels it would replace
+    are measured faster (narrow layers, row-major weights on a shape the NZ prefill kernel does not take) the query is
+    theirs: none."""
+    L, n = q.abi(), ctypes.c_size_t(0)
+    for M, N, K, code, group, mid in [
+        (23, 11008, 4096, q.QK_I8_NK, 0, True),
+        (24, 1536, 5120, q.QK_I8_NK, 0, False),
+        (20, 4096, 4096, q.QK_I8_NK, 128, False),
+        (40, 4096, 4096, q.QK_I8_NK, 128, True),
+        (48, 1536, 5120, q.QK_I8_NZ, 128, False),
+        (48, 1536, 5120, q.QK_I4_NZ, 128, False),
+        (77, 3072, 2048, q.QK_I8_NK, 0, False),
+        (400, 13696, 5120, q.QK_I8, 0, False),
+        (300, 13696, 5120, q.QK_I8, 0, True),
+        (600, 3072, 2048, q.QK_I32, 128, False),
+        (256, 32000, 4096, q.QK_I32, 128, True),
+    ]:
+        assert L.qk_weight_quant_bmm_workspace_size(M, N, K, code, group, ctypes.byref(n)) == 0
+        assert (n.value > 0) == mid, (M, N, K, code, n.value)
+
+
 def test_w8a8_split_plan_workspace_sizes():
     """The K-split plans' workspaces (host arithmetic only).  cfg5's down projection (512 x 4096 x 14336) has 32
     tiles of 256 x 256, split 8 ways to fill the CUs; on 128-row tiles it has 64, split 4 ways: half the int32
