@@ -927,7 +927,7 @@ __global__ __launch_bounds__(nzg::NT) void w4nz_gemm(WqbmmArgs p, int tiles_m, i
 // 1 beyond; int8 (two loads per block), 3 up to 2 superblocks, 2 for 3, 1 beyond.  Only these
 // (NB, NIT) pairs are built.
 constexpr int nz_max_blocks(int nit, bool w8) {
-    if (nit == 0) return w8 ? 3 : 4;  // the ragged form keeps two superblocks in registers, whatever its length
+    if (nit == 0) return w8 ? 3 : 4;  // the ragged form keeps two (up to 4 rows: three or four) superblocks in registers
     return w8 ? (nit <= 2 ? 3 : nit == 3 ? 2 : 1) : (nit <= 3 ? 4 : nit == 4 ? 3 : nit == 5 ? 2 : 1);
 }
 

@@ -1720,11 +1720,10 @@ bool big_nk_full(const QmmArgs& p, int nsplit) {
            p.sbn < (1 << 24) && (uintptr_t)p.epi.out % 16 == 0 && p.epi.ldo % 8 == 0;
 }
 
-// The direct-to-LDS kernel (any M: a ragged last row tile reads zeros past M and stores only its rows): K
-// ranges of whole 4-stage rings, 16-byte aligned rows, and every operand range of a tile addressable by a
-// 32-bit buffer offset.
-bool big_dma_ok(const QmmArgs& p, bool b_kn, int nsplit) {
-    (void)nsplit;
+// The direct-to-LDS kernel (any M: a ragged last row tile reads zeros past M and stores only its rows; any N of whole
+// 16-byte pieces, 8 columns on [N,K]; any K of whole 16-byte chunks, in any number of splits): 16-byte aligned rows, and
+// every operand range of a tile addressable by a 32-bit buffer offset.
+bool big_dma_ok(const QmmArgs& p, bool b_kn) {
     return plan_override().qmm_dma && p.K > 0 && p.K % 16 == 0 && p.lda < (1 << 24) && p.sbk < (1 << 24) &&
            p.sbn < (1 << 24) && p.lda % 16 == 0 && (uintptr_t)p.a % 16 == 0 && (uintptr_t)p.b % 16 == 0 &&
            (uintptr_t)p.epi.out % 16 == 0 && p.epi.ldo % 8 == 0 &&
@@ -1747,7 +1746,7 @@ hipError_t launch_big(const QmmArgs& p, bool b_kn, int tiles_m, int tiles_n, int
                       hipStream_t stream) {
     const dim3 grid((uint32_t)(tiles_m * tiles_n * nsplit));
     const bool full = big_nk_full(p, nsplit) && p.M % big::BM == 0;  // the register-staged kernel's whole tiles
-    const bool dma = big_dma_ok(p, b_kn, nsplit);
+    const bool dma = big_dma_ok(p, b_kn);
     if (nsplit > 1 && !full && !dma) return hipErrorInvalidValue;  // not planned (launch_quant_matmul unsplits)
     if (dma) {
         const auto k = dma_ragged(p, nsplit) ? (b_kn ? qmm_dma<kLayKN, OUT, 256, true> : qmm_dma<kLayNK, OUT, 256, true>)
@@ -2023,9 +2022,8 @@ size_t mid_workspace(const MidPlan& m) {
 // (K = 11008, N = 4096, M = 70-128: qmm_mid 22-23 us, 8 splits 24.4-25.8; K = 8192, N = 3584: 17.1-17.7 against
 // 19.8-20.4; K = 13696, N = 5120, M = 100: 37.0 against 31.8; four rounds, K = 4096, N = 28672, M = 90: 52.1
 // against 40.5).  The sums are exact, so the bits equal qmm_mid's.  Returns the split count, or 0 for qmm_mid.
-constexpr double kMidHbmKn = 3.1e6, kMidHbmNz = 4.6e6;  // qmm_mid's weight read rate, bytes per us
-
-int small_split(int64_t M, int64_t N, int64_t K, const MidPlan& mp, double mid_hbm = kMidHbmKn) {
+int small_split(int64_t M, int64_t N, int64_t K, const MidPlan& mp, bool nz = false) {
+    const double mid_hbm = nz ? 4.6e6 : 3.1e6;  // qmm_mid's weight read rate, bytes per us
     const PlanOverride& ov = plan_override();  // debug override: qmm_small=0 never, =<n> that split count
     if (ov.qmm_small == 0 || mp.bm == 0 || M <= 32 || M > 128 || N % 16 != 0 || K <= 0) return 0;
     auto rounds = [](int64_t wgs) { return (double)((wgs + 255) / 256); };
@@ -2034,7 +2032,7 @@ int small_split(int64_t M, int64_t N, int64_t K, const MidPlan& mp, double mid_h
     const double t_mid_fill = rounds((int64_t)mp.tiles * mp.nsplit) * (mp.bm + mp.bn) * (double)(K / mp.nsplit) / kFill;
     const double t_mid = t_mid_fill > w_bytes / mid_hbm ? t_mid_fill : w_bytes / mid_hbm;
     int best = 0;
-    double t_best = (mid_hbm == kMidHbmNz && mp.tiles <= 512 ? 0.82 : 0.9) * t_mid;
+    double t_best = (nz && mp.tiles <= 512 ? 0.82 : 0.9) * t_mid;
     for (int ns : {2, 4, 8}) {
         if (ov.qmm_small > 0 && ns != ov.qmm_small) continue;
         if (K / ns < 256 || (ns - 1) * dma_k_len(K, ns) >= K) continue;
@@ -2156,7 +2154,7 @@ hipError_t launch_quant_matmul(const QmmArgs& p, void* workspace, size_t ws_byte
         if (b_kn16) {  // wide or deep [K,N] weights: 128-row K splits where the cost model favours them
             if (const int ns = small_split(p.M, p.N, p.K, mp)) {
                 const BigPlan sb = small_split_plan(p.M, p.N, ns);
-                if (big_dma_ok(p, true, ns) && partial && ws_bytes >= big_split_workspace(sb, p.M, p.N) &&
+                if (big_dma_ok(p, true) && partial && ws_bytes >= big_split_workspace(sb, p.M, p.N) &&
                     (uintptr_t)partial % 16 == 0)
                     return launch_split128<kLayKN>(p, sb, partial, stream);
             }
@@ -2192,15 +2190,15 @@ hipError_t launch_quant_matmul(const QmmArgs& p, void* workspace, size_t ws_byte
     if (big_ok && bp.bm == 128) {
         // the 128-row split needs the direct-to-LDS kernel and its workspace; otherwise the shape runs unsplit
         const size_t need = big_split_workspace(bp, p.M, p.N);
-        if (big_dma_ok(p, b_kn, bp.nsplit) && partial && ws_bytes >= need && (uintptr_t)partial % 16 == 0)
+        if (big_dma_ok(p, b_kn) && partial && ws_bytes >= need && (uintptr_t)partial % 16 == 0)
             return b_kn ? launch_split128<kLayKN>(p, bp, partial, stream) : launch_split128<kLayNK>(p, bp, partial, stream);
         bp = big_plan(p.M, p.N, p.K, false);
     }
     // a ragged split runs only on the direct-to-LDS kernel; otherwise the tiled kernels take the shape
-    if (big_ok && bp.ragged && bp.nsplit > 1 && !big_dma_ok(p, b_kn, bp.nsplit)) big_ok = false;
+    if (big_ok && bp.ragged && bp.nsplit > 1 && !big_dma_ok(p, b_kn)) big_ok = false;
     // a split of a ragged M runs only on the direct-to-LDS kernel; otherwise the register-staged kernel runs
     // the shape unsplit (the planned workspace is then unused)
-    if (big_ok && bp.nsplit > 1 && big_dma_ok(p, b_kn, bp.nsplit)) bp.nsplit = dma_splits(p.K, bp.nsplit);
+    if (big_ok && bp.nsplit > 1 && big_dma_ok(p, b_kn)) bp.nsplit = dma_splits(p.K, bp.nsplit);
     else if (big_ok && bp.nsplit > 1 && p.M % big::BM != 0) bp.nsplit = 1;
     if (big_ok && bp.nsplit > 1) {
         // splits need whole aligned tiles and the workspace; otherwise the tiled kernels take the shape
@@ -2232,8 +2230,9 @@ hipError_t launch_quant_matmul(const QmmArgs& p, void* workspace, size_t ws_byte
 // ---------------------------------------------------------------------------
 // W8A8 on an int8 NZ weight (p.b: [N/16][K/64][64][16]; p.sbk and p.sbn unused).  By shape: M <= 16 the
 // decode stream qmm_nzd (no workspace); the mid-M plan qmm_mid on NZ blocks (64-column blocks, no split);
-// 256-column tiles (any M) qmm_dma on NZ blocks (a K split as planned for the row-major weight); any other
-// shape unpacks the weight to [K,N] in the workspace and runs the row-major kernels on it:
+// 256-column tiles (any M, N and K) qmm_dma on NZ blocks (a K split as planned for the row-major weight); a shape of too
+// few tiles for whole ones and too short a K to split (M = 300, N = 1024, K = 512) unpacks the weight to [K,N] in the
+// workspace and runs the row-major kernels on it:
 // [ND weight, 256-byte rounded][that call's workspace].  The C ABI guarantees 16-byte aligned x1 rows
 // (row stride below 2^24), weight and output.
 namespace {
@@ -2272,8 +2271,8 @@ hipError_t launch_nzd(const QmmArgs& p, const NzdPlan& z, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// qmm_dma on NZ blocks: every shape with a plan (any M, N and K; the last column tile and the last K range of an
-// NZ weight may be ragged)
+// qmm_dma on NZ blocks: every shape that big_plan has a plan for (any M, N and K; the last column tile and the last K
+// range of an NZ weight may be ragged; no plan below 192 tiles where K / 2 is under 512)
 bool nz_dma_ok(const BigPlan& b) { return plan_override().qmm_dma && b.ok; }
 
 BigPlan nz_big_plan(int64_t M, int64_t N, int64_t K) {
@@ -2299,7 +2298,7 @@ size_t quant_matmul_nz_workspace(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     if (nzd_plan(M, N, K).nb) return 0;
     if (mid_plan(M, N, K, false).bm) {  // the mid-M shapes: qmm_mid on NZ blocks (no workspace) or split tiles
-        const int ns = small_split(M, N, K, mid_plan(M, N, K, false), kMidHbmNz);
+        const int ns = small_split(M, N, K, mid_plan(M, N, K, false), true);
         return ns ? big_split_workspace(small_split_plan(M, N, ns), M, N) : 0;
     }
     const BigPlan b = nz_big_plan(M, N, K);
@@ -2317,7 +2316,7 @@ hipError_t launch_quant_matmul_nz(const QmmArgs& p, void* workspace, size_t ws_b
     if (mp.bm) {
         // wide or deep weights: 128-row K-split tiles where the cost model favours them (a workspace smaller
         // than the query's runs qmm_mid, the same bits)
-        if (const int ns = small_split(p.M, p.N, p.K, mp, kMidHbmNz)) {
+        if (const int ns = small_split(p.M, p.N, p.K, mp, true)) {
             const BigPlan sb = small_split_plan(p.M, p.N, ns);
             if (plan_override().qmm_dma && ws && ws_bytes >= big_split_workspace(sb, p.M, p.N) &&
                 (uintptr_t)ws % 16 == 0)
